@@ -90,40 +90,100 @@ __global__ __launch_bounds__(256) void fa_combine_kernel(const float *__restrict
     }
 }
 
-// The same merge for many rows and few splits (prefill): 64 threads per row,
-// one float4 of the row each, 4 rows per block; every thread walks the splits
-// itself (the (m, l) pairs are the same for the 64 threads of a row and come
-// from the cache).
-constexpr int kRowsMaxSplits = 32;
+// The same merge for many rows (prefill): WPR wavefronts per row, a float4 of
+// the row per lane. Lane s first reads the (m, l) pair of split s (one load per
+// 64 splits), takes the row's maximum and its split's weight; the partials are
+// then read kBatch splits at a time, only those of nonzero weight: a split in
+// which the row sees no key (m = -inf) has left its acc unwritten. With WPR = 4
+// wavefront w takes splits w, w + 4, ... and the four sums meet in LDS.
+// Bound by the partials' bytes, its launch and two memory latencies. 592 rows x
+// 40 splits (24 MB): 16.8 us in the kernel above (16 blocks per row, 64 bytes of
+// a partial at a time), 7.4 us here at 42 splits; 8192 rows x 4 splits (33 MB):
+// 8.0 us with every thread walking the splits' pairs by itself, 8.4 us here.
+constexpr int kBatch = 4;
+constexpr int kRowsMin = 256;
+constexpr int kRowsOneWaveSplits = 8;
+template <int WPR>
 __global__ __launch_bounds__(256) void fa_combine_rows_kernel(const float *__restrict__ part_acc,
                                                               const float *__restrict__ part_ml,
                                                               int n_splits, int rows_total,
                                                               float *__restrict__ dst, const char *gate,
                                                               int64_t gate_nb1, int64_t gate_nb2, int H) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    constexpr int kW = kMaxSplits / 64;  // splits per lane
+    __shared__ float4 xo[WPR > 1 ? 4 : 1][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = threadIdx.x & 63;
-    if (row >= rows_total) return;
-    float ms[kRowsMaxSplits];
-    float M = -INFINITY;
-#pragma unroll
-    for (int sp = 0; sp < kRowsMaxSplits; ++sp) {
-        ms[sp] = sp < n_splits ? part_ml[((int64_t)sp * rows_total + row) * 2] : -INFINITY;
-        M = fmaxf(M, ms[sp]);
-    }
+    const int row = WPR > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
+    if (row >= rows_total) return;  // whole wavefronts; with WPR > 1 the grid is rows_total
+    const float2 *pm = reinterpret_cast<const float2 *>(part_ml) + row;
+    const int n_w = (n_splits + 63) >> 6;
     const int64_t sstride = (int64_t)rows_total * 256;
     const float *pa = part_acc + (int64_t)row * 256 + 4 * c;
-    float L = 0.0f;
+    // the first batch is on its way before the weights are known (what an
+    // unwritten partial holds is never used: its weight is 0)
+    float4 a[kBatch];
+    const int w0 = WPR > 1 ? wave : 0;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+        const int sp = w0 + WPR * j;
+        a[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (sp < n_splits) a[j] = *reinterpret_cast<const float4 *>(pa + sp * sstride);
+    }
+    float2 ml[kW];
+    float M = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+        const int sp = 64 * k + c;
+        ml[k] = k < n_w && sp < n_splits ? pm[(int64_t)sp * rows_total] : make_float2(-INFINITY, 0.0f);
+        M = fmaxf(M, ml[k].x);
+    }
+#pragma unroll
+    for (int o = 1; o <= 8; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    M = fmaxf(M, lane_xor16(M));
+    M = fmaxf(M, lane_xor32(M));
+    float w[kW], L = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+        w[k] = ml[k].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ml[k].x - M) * kLog2e);
+        L = fmaf(ml[k].y, w[k], L);
+    }
+#pragma unroll
+    for (int o = 1; o <= 8; o <<= 1) L += __shfl_xor(L, o);
+    L += lane_xor16(L);
+    L += lane_xor32(L);
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int sp = 0; sp < kRowsMaxSplits; ++sp) {
-        if (sp >= n_splits) break;
-        const float w = (M == -INFINITY || ms[sp] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((ms[sp] - M) * kLog2e);
-        L = fmaf(part_ml[((int64_t)sp * rows_total + row) * 2 + 1], w, L);
-        const float4 a = *reinterpret_cast<const float4 *>(pa + sp * sstride);
-        o.x = fmaf(a.x, w, o.x);
-        o.y = fmaf(a.y, w, o.y);
-        o.z = fmaf(a.z, w, o.z);
-        o.w = fmaf(a.w, w, o.w);
+    for (int k = 0; k < kW; ++k) {
+        if (k >= n_w) break;
+        const int end = n_splits - 64 * k < 64 ? n_splits - 64 * k : 64;
+        for (int s0 = w0; s0 < end; s0 += WPR * kBatch) {
+            float wt[kBatch];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int sp = s0 + WPR * j;
+                wt[j] = sp < end ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[k]), sp)) : 0.0f;
+                if (64 * k + s0 != w0 && wt[j] != 0.0f)
+                    a[j] = *reinterpret_cast<const float4 *>(pa + (64 * k + sp) * sstride);
+            }
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                if (wt[j] == 0.0f) continue;
+                o.x = fmaf(a[j].x, wt[j], o.x);
+                o.y = fmaf(a[j].y, wt[j], o.y);
+                o.z = fmaf(a[j].z, wt[j], o.z);
+                o.w = fmaf(a[j].w, wt[j], o.w);
+            }
+        }
+    }
+    if (WPR > 1) {
+        xo[wave][c] = o;
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int j = 1; j < 4; ++j) {
+            const float4 a = xo[j][c];
+            o.x += a.x, o.y += a.y, o.z += a.z, o.w += a.w;
+        }
     }
     const float inv = L == 0.0f ? 0.0f : 1.0f / L;
     float r[4] = {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
@@ -145,8 +205,14 @@ int launch_fa_combine(const float *part_acc, const float *part_ml, int n_splits,
     if (n_splits > kMaxSplits)
         return set_error(SQA_ERR_UNSUPPORTED, "fa_combine: %d splits > %d", n_splits, kMaxSplits);
     const int prof = profile_start("fa_combine", s);
-    if (n_splits <= kRowsMaxSplits && rows_total >= 64) {
-        fa_combine_rows_kernel<<<dim3((unsigned)((rows_total + 3) / 4)), dim3(256), 0, s>>>(
+    // Few rows (decode, verify, the smallest chunks) need the 16 blocks per row of
+    // the first kernel to fill the chip; from kRowsMin rows on, one block or a
+    // quarter of one per row does, and reads 1 KB of a partial at a time.
+    if (rows_total >= kRowsMin && n_splits <= kRowsOneWaveSplits) {
+        fa_combine_rows_kernel<1><<<dim3((unsigned)((rows_total + 3) / 4)), dim3(256), 0, s>>>(
+            part_acc, part_ml, n_splits, rows_total, dst, g, g1, g2, H);
+    } else if (rows_total >= kRowsMin) {
+        fa_combine_rows_kernel<4><<<dim3((unsigned)rows_total), dim3(256), 0, s>>>(
             part_acc, part_ml, n_splits, rows_total, dst, g, g1, g2, H);
     } else {
         fa_combine_kernel<<<dim3((unsigned)rows_total, 16), dim3(256), 0, s>>>(part_acc, part_ml, n_splits,

@@ -459,6 +459,7 @@ struct PrefillParams {
     const int32_t *tile_lim;  // with a mask: [q_tiles] exclusive key limit of each query tile
     int n_splits;
     int q_tiles;        // workgroups per (KV head, split)
+    bool skew;          // order of the workgroups, see the kernel
     int64_t split_len;  // keys per split, a multiple of kPK
     int qb;             // query positions per workgroup (128 / G)
     int mask_stage;     // LDS bytes per mask stage (qb x 64)
@@ -479,12 +480,25 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
     // Renumber so that each XCD gets a contiguous run of ids, i.e. the query
     // tiles of the same (KV head, split): they stream the same K/V range, which
     // that XCD's L2 then serves to all of them.
+    // With p.skew (a causal chunk whose query tiles see ranges of very different
+    // length) such runs would give whole XCDs the long tiles. The workgroups then
+    // go out longest first: split by split (the early ones are seen whole), the
+    // last query tile first, neighbours on different XCDs.
     const int nb = (int)gridDim.x;
     const int lin = (int)blockIdx.x;
-    const int id = nb % 8 == 0 ? (lin % 8) * (nb / 8) + lin / 8 : lin;
-    const int q_tile = id % p.q_tiles;
-    const int grp = id / p.q_tiles;
-    const int kvh = grp / p.n_splits, split = grp % p.n_splits;
+    const int x = lin & 7, per = nb >> 3, rem = nb & 7;
+    int q_tile, kvh, split;
+    if (p.skew) {
+        const int wgs = p.q_tiles * p.Hkv, r = lin % wgs;
+        split = lin / wgs;
+        q_tile = p.q_tiles - 1 - r / p.Hkv;
+        kvh = r % p.Hkv;
+    } else {
+        const int id = x * per + (x < rem ? x : rem) + (lin >> 3), grp = id / p.q_tiles;
+        q_tile = id % p.q_tiles;
+        kvh = grp / p.n_splits;
+        split = grp % p.n_splits;
+    }
     const int q_base = q_tile * p.qb;
 
     // Key range: the split, cut at the last key any query of the workgroup sees.
@@ -499,6 +513,17 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         if (k_end > lim) k_end = lim;
     }
     const int n_tiles = k_end > k_begin ? (int)((k_end - k_begin + kPK - 1) / kPK) : 0;
+    if (n_tiles == 0 && p.n_splits > 1) {
+        // a split past the tile's last visible key leaves its O unwritten: the
+        // merge takes no partial whose m is -inf
+        const int pos = q_base + tid / p.G;
+        if (tid < kRowsPerWG && pos < p.n_q) {
+            const int64_t row = (int64_t)split * p.n_q * p.H + (int64_t)pos * p.H + kvh * p.G + tid % p.G;
+            store_through(p.part_ml + row * 2, -INFINITY);
+            store_through(p.part_ml + row * 2 + 1, 0.0f);
+        }
+        return;
+    }
 
     // ---------------- DMA: 1 KB per instruction, a fixed share per wave ---------
     // Iteration t: K half + mask of tile t + 1, V half of tile t (stage = tile & 1).
@@ -944,6 +969,93 @@ struct PrefillPlan {
     size_t off_kv, off_dvmax, off_qh, off_ql, off_mask, off_lim, off_pa, off_pm, total;
 };
 
+// Key splits of a chunk. A workgroup fills a CU (LDS), so the workgroups of one
+// split (wgs = q_tiles per KV head) run in rounds of one per CU. Up to an eighth
+// of the CUs, whole splits fill a round to 8/9 or more; with more workgroups
+// per split, up to kMaxRounds rounds let a later one fill what a single round
+// leaves idle (160 workgroups: 2 rounds of 3 splits instead of 2 of 2).
+// Up to kOneSplitKeys keys a chunk stays whole: its output and gate leave in the
+// attention kernel's epilogue, with no partials and no merge.
+constexpr int kMinSplitTiles = 2;  // 64 keys
+constexpr int kMaxRounds = 4;
+constexpr int kOneSplitKeys = 512;
+int64_t max_splits(int64_t n_kv, int64_t wgs) {
+    if (n_kv <= kOneSplitKeys) return 1;
+    const int64_t cus = device_cu_count();
+    const int64_t by_len = ((n_kv + kPK - 1) / kPK + kMinSplitTiles - 1) / kMinSplitTiles;
+    const int64_t by_rounds = (8 * wgs > cus ? kMaxRounds : 1) * cus / wgs;
+    int64_t s = by_len < by_rounds ? by_len : by_rounds;
+    if (s > kMaxSplits) s = kMaxSplits;
+    return s < 1 ? 1 : s;
+}
+
+// Keys per split, a multiple of kPK: the candidate of least estimated time, in
+// units of one tile of one workgroup. Measured: 2.2 us with the chip full, down to
+// 0.75 of that with few CUs busy; a workgroup costs about kWgTiles tiles beside
+// its own (start, Q rows, fill and drain, output), the merge kMergeTiles plus
+// kMergeRow per row and split (1 KB written and read). The chunk is taken as
+// causal and the last n_q keys as its own (a mask or a position may say
+// otherwise: the estimate is then off, the result not). Workgroups that see no
+// key leave at once; of the others, in dispatch order, round k starts with
+// workgroup k * CUs and is taken to last as long as that one. Splitting at all
+// must be worth kMargin: the estimate is no better than that. us per call (16
+// heads on 2, pre-passes and merge included) with ceil(CUs / wgs) splits of 512
+// keys or more, with this choice, and with the best split count of all tried:
+//   37 queries on 20048 keys    75.0  65.1
+//   300 on 3301                 94   65   64 (7 splits were 266 workgroups)
+//   600 on 20600               610  432  426
+//   405 on 171568             4390 2331
+//   1280 on 6280               401  297  293
+//   2048 on 2048               145  145  128 (2 splits)
+constexpr float kWgTiles = 2.0f, kMergeTiles = 2.0f, kMergeRow = 1.2e-4f, kMargin = 0.98f;
+float tile_time(float busy) { return 0.75f + 0.25f * busy; }  // busy: share of the CUs
+bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
+int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q_tiles, int64_t rows) {
+    const int64_t cus = device_cu_count(), wgs = q_tiles * Hkv;
+    const int64_t tiles = (n_kv + kPK - 1) / kPK, most = max_splits(n_kv, wgs);
+    // key tiles that query tile i sees: first + i * step, at most all
+    const float step = (float)qb / kPK;
+    const float first = ((float)(n_kv > n_q ? n_kv - n_q : 0) + (float)qb) / kPK;
+    int64_t best_len = tiles, last_len = 0;
+    float best = INFINITY;
+    for (int64_t s = 1; s <= most; ++s) {
+        const int64_t len = (tiles + s - 1) / s;
+        if (len == last_len) continue;
+        last_len = len;
+        const int64_t n_s = (tiles + len - 1) / len;
+        float t = 0.0f, last = 0.0f;  // estimate, its last round
+        int64_t next = 0;             // first workgroup of the next round
+        auto round = [&](float n) {
+            last = n + kWgTiles;
+            t += last;
+            next += cus;
+        };
+        // the splits that every query tile sees whole, then the others one by one
+        int64_t j = (int64_t)(first / (float)len);
+        if (j > n_s - 1) j = n_s - 1;
+        int64_t live = j * wgs;  // workgroups with keys
+        float work = (float)(live * len);
+        while (next < live) round((float)len);
+        for (; j < n_s; ++j) {
+            const float at = (float)(j * len);
+            // query tiles i0 .. q_tiles - 1 reach into it, the last one furthest
+            const int64_t i0 = first > at ? 0 : (int64_t)((at - first) / step) + 1;
+            if (i0 >= q_tiles) break;
+            const float all = (float)(j == n_s - 1 ? tiles - j * len : len);
+            const float lo = first + (float)i0 * step - at, hi = first + (float)(q_tiles - 1) * step - at;
+            const int64_t here = (q_tiles - i0) * Hkv;
+            while (next < live + here) round(fminf(all, hi - (float)((next - live) / Hkv) * step));
+            live += here;
+            work += (float)here * (lo >= all ? all : 0.5f * (lo + fminf(hi, all)));
+        }
+        const float part = live > cus ? (float)(live - (next - cus)) / (float)cus : work / ((float)cus * (last - kWgTiles));
+        t += last * (tile_time(fminf(part, 1.0f)) - 1.0f);
+        t = n_s > 1 ? t + kMergeTiles + kMergeRow * (float)(n_s * rows) : kMargin * t;
+        if (t < best) best = t, best_len = len;
+    }
+    return best_len * kPK;
+}
+
 PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     PrefillPlan pl{};
     const int G = (int)(H / Hkv);
@@ -951,15 +1063,11 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     pl.mask_stage = pl.qb * kPK * 2;
     pl.kv_tiles = (n_kv + 63) / 64 * 2;  // vdeq writes 64-key groups
     pl.q_tiles = (int)((n_q + pl.qb - 1) / pl.qb);
-    const int64_t wgs = (int64_t)pl.q_tiles * Hkv;
-    const int64_t cus = device_cu_count();
-    int64_t splits = (cus + wgs - 1) / wgs;
-    const int64_t max_by_len = (n_kv + 511) / 512;  // at least ~512 keys per split
-    if (splits > max_by_len) splits = max_by_len;
-    if (splits > kMaxSplits) splits = kMaxSplits;
-    if (splits < 1) splits = 1;
-    pl.split_len = ((n_kv + splits - 1) / splits + kPK - 1) / kPK * kPK;
+    pl.split_len = split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H);
     pl.n_splits = (int)((n_kv + pl.split_len - 1) / pl.split_len);
+    // partials: for the most splits that a cache of up to n_kv keys can get, so
+    // that a workspace sized for a longer cache serves every shorter one
+    const int64_t parts = max_splits(n_kv, pl.q_tiles * Hkv);
     size_t o = 0;
     pl.off_kv = o; o = al256(o + (size_t)Hkv * pl.kv_tiles * kTileBytes);
     pl.off_dvmax = o; o = al256(o + (size_t)Hkv * 4);
@@ -969,10 +1077,10 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     pl.off_lim = o; o = al256(o + (size_t)pl.q_tiles * 4);
     pl.off_pa = o;
     pl.off_pm = o;
-    if (pl.n_splits > 1) {
-        o = al256(o + (size_t)pl.n_splits * n_q * H * kHeadDim * 4);
+    if (parts > 1) {
+        o = al256(o + (size_t)parts * n_q * H * kHeadDim * 4);
         pl.off_pm = o;
-        o = al256(o + (size_t)pl.n_splits * n_q * H * 2 * 4);
+        o = al256(o + (size_t)parts * n_q * H * 2 * 4);
     }
     pl.total = o + 256;
     return pl;
@@ -1068,6 +1176,7 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     p.n_splits = pl.n_splits;
     p.q_tiles = pl.q_tiles;
     p.split_len = pl.split_len;
+    p.skew = skewed(n_q, n_kv);
     p.qb = pl.qb;
     p.mask_stage = pl.mask_stage;
     p.part_acc = reinterpret_cast<float *>(base + pl.off_pa);

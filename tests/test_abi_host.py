@@ -92,6 +92,18 @@ def test_workspace_size_scales_with_splits(sqa):
     assert big <= 256 * 16 * 258 * 4 + 172032 * 2 + 4 * 256
 
 
+@pytest.mark.parametrize("n_q", [5, 37, 300, 512, 1280, 2048])
+def test_prefill_workspace_of_a_longer_cache_serves_a_shorter_one(sqa, n_q):
+    """A workspace is sized once for the longest context: whatever the split plan
+    does at a shorter one must fit."""
+    L, last = sqa.lib(), 0
+    for n_kv in list(range(32, 4096, 96)) + [8192, 20048, 65536, 65568, 172032]:
+        q, k, o = fa_descs(sqa, n_q=n_q, n_kv=n_kv)
+        need = L.sqa_flash_attn_ext_workspace_size(ctypes.byref(q), ctypes.byref(k), ctypes.byref(k), ctypes.byref(o))
+        assert need >= last > -1
+        last = need
+
+
 class FakeKv:
     """KvCache bookkeeping with dummy (never dereferenced) buffer addresses."""
 

@@ -244,3 +244,32 @@ def test_mask_form_start_chunk_costs_what_the_causal_form_does(sqa, orc, dev):
     print(f"start chunk 512x512: fa_prefill mask form {1e3 * med['mask']:.2f} us, "
           f"causal form {1e3 * med['causal']:.2f} us")
     assert med["mask"] <= 1.10 * med["causal"]
+
+
+@pytest.mark.parametrize("n_q,n_kv,q_pos0,H,Hkv", [
+    (513, 513, 0, 16, 2),      # just past one split; most query tiles do not reach the last splits
+    (15, 700, 685, 16, 2),     # 240 rows and
+    (16, 700, 684, 16, 2),     # 256 rows: the two forms of the merge
+    (300, 3301, 3001, 16, 2),  # a round that one split more would overfill
+    (700, 1300, 600, 16, 4),   # skewed, several rounds
+    (1280, 2000, 720, 16, 2),  # more than one round of workgroups per split
+    (40, 1500, 0, 16, 2),      # rows that end far before the cache does: whole splits without a key
+    (600, 600, 0, 4, 4),       # 128 positions per query tile
+])
+def test_prefill_split_plan(sqa, orc, dev, n_q, n_kv, q_pos0, H, Hkv):
+    """Split counts, dispatch orders and merges of the plan, with the workspace
+    holding NaN bytes: a split that sees no key writes no partial."""
+    q, kq, vq = qkv(orc, n_q + n_kv, n_q, n_kv, H=H, Hkv=Hkv)
+    rows = np.unique(np.r_[0:n_q:max(1, n_q // 24), n_q - 1])
+    ref = np.concatenate([orc.flash_attn_ext_causal(q[r:r + 1], kq, vq, q_pos0 + int(r)) for r in rows])
+    qd, kd, vd = (torch.from_numpy(x).to(dev) for x in (q, kq, vq))
+    mask = torch.from_numpy(orc.causal_mask(n_q, n_kv, q_pos0)).to(dev)
+    for form in ("causal", "mask"):
+        ws = torch.full((sqa.flash_attn_workspace_size(qd, kd, n_kv),), 0xFF, dtype=torch.uint8, device=dev)
+        if form == "causal":
+            got = sqa.flash_attn_ext_causal(qd, kd, vd, n_kv, q_pos0, workspace=ws)
+        else:
+            got = sqa.flash_attn_ext(qd, kd, vd, n_kv, mask=mask, workspace=ws)
+        err = rel_err(got.cpu().numpy()[rows], ref)
+        print(f"split plan {form} n_q={n_q} n_kv={n_kv} at {q_pos0}: max err / rms = {err:.3e}")
+        assert err <= TOL
