@@ -4,7 +4,9 @@ Python host mirror of the C ABI in include/sqattn.h, named after the ggml ops
 and the engine objects it stands in for (reference: src/backend/ffi.rs:363-405,
 src/engine/kv.rs). Device memory and streams come from PyTorch; every kernel
 runs from libsqattn.so, which sits next to this file. If the library is
-missing the import fails: there is no CPU fallback.
+missing the import fails: there is no CPU fallback. Calls that give their output
+and workspace and use the current stream go through _sqahost.so
+(binding/host.cpp), the others build their descriptors here.
 
 Tensor conventions (torch shapes, C order, all on the GPU):
   q       float32 (n_q, H, D)             the engine's [D, H, n_q] Q
@@ -13,6 +15,8 @@ Tensor conventions (torch shapes, C order, all on the GPU):
   out     float32 (n_q, H, D)             [D, H, n_q] attention output
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import struct
 import os
 
@@ -27,6 +31,7 @@ __all__ = [
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libsqattn.so")
+HOST_PATH = os.path.join(HERE, "_sqahost.so")
 
 TYPE_F32, TYPE_F16, TYPE_Q4_0, TYPE_Q4_K, TYPE_I32, TYPE_I64 = 0, 1, 2, 12, 26, 27
 Q4_K_BLOCK = 144  # bytes per 256-value Q4_K super-block
@@ -147,6 +152,22 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def _load_host():
+    """The native binding of the hot entry points (raises if it was never built)."""
+    global _host
+    lib()  # the binding links against the library beside it
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f"{HOST_PATH} is missing: run __graft_entry__.build() first")
+    loader = importlib.machinery.ExtensionFileLoader("_sqahost", HOST_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_sqahost", loader))
+    loader.exec_module(mod)
+    _host = mod
+    return mod
+
+
 def last_error():
     return lib().sqa_last_error().decode()
 
@@ -207,6 +228,12 @@ def set_rows_q4_0(cache, src, idx, stream=None):
     """cache[idx[i]] = quantize_row_q4_0(src[i]) (GGML_OP_SET_ROWS, kv.rs:356-396).
 
     cache: uint8 (rows, ..., row_bytes) contiguous; src: float32 (n, ne0); idx: int64 (n,)."""
+    if stream is None:
+        rc = (_host or _load_host()).set_rows(cache, src, idx)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return cache
     rows = cache.shape[0]
     rb = cache[0].numel()
     ne0 = src.shape[1]
@@ -233,6 +260,12 @@ def rope_norm_set_rows_q4_0(cache, src, norm_w, eps, pos, rope, idx, stream=None
     cache: uint8 (rows, ..., n_head*D//32*18) contiguous; src: float32 (n_tok, n_head, D)
     with contiguous rows; norm_w: float32 (D,) or None; pos: int32 (4*n_tok,);
     idx: int64 (n_tok,)."""
+    if stream is None and idx is not None:
+        rc = (_host or _load_host()).rope_norm(cache, src, norm_w, eps, pos, rope, idx)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return cache
     n_tok, n_head, D = src.shape
     rows = cache.shape[0]
     rb = cache[0].numel()
@@ -247,6 +280,12 @@ def rope_norm_set_rows_q4_0(cache, src, norm_w, eps, pos, rope, idx, stream=None
 
 def rope_norm_f32(out, src, norm_w, eps, pos, rope, stream=None):
     """Q producer (reference attn.rs:166-199): out float32 (n_tok, n_head, D) contiguous."""
+    if stream is None:
+        rc = (_host or _load_host()).rope_norm(out, src, norm_w, eps, pos, rope, None)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return out
     n_tok, n_head, D = src.shape
     ts, tw, tp = _producer_descs(src, norm_w, pos)
     to = Tensor.make(TYPE_F32, [D, n_head, n_tok], [4, D * 4, n_head * D * 4], out.data_ptr())
@@ -283,6 +322,12 @@ def _workspace(nbytes, device):
 def flash_attn_ext(q, k_cache, v_cache, n_kv, mask=None, scale=None, max_bias=0.0, softcap=0.0,
                    out=None, workspace=None, stream=None):
     """ggml_flash_attn_ext(q, k, v, mask, scale, max_bias, softcap) over q4_0 caches."""
+    if stream is None and out is not None and workspace is not None:
+        rc = (_host or _load_host()).fa(q, k_cache, v_cache, n_kv, mask, scale, max_bias, softcap, out, workspace)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return out
     n_q, H, D = q.shape
     scale = D ** -0.5 if scale is None else scale
     if out is None:
@@ -318,6 +363,12 @@ def flash_attn_ext_static(q, k_cache, v_cache, n_kv, mask=None, scale=None, max_
 def flash_attn_ext_causal(q, k_cache, v_cache, n_kv, q_pos0, gate=None, scale=None, out=None,
                           workspace=None, stream=None):
     """Mask-free causal FA (query t at position q_pos0 + t) with optional fused sigmoid gate."""
+    if stream is None and out is not None and workspace is not None:
+        rc = (_host or _load_host()).fa_causal(q, k_cache, v_cache, n_kv, q_pos0, gate, scale, out, workspace)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return out
     n_q, H, D = q.shape
     scale = D ** -0.5 if scale is None else scale
     if out is None:
@@ -368,6 +419,12 @@ def out_proj_workspace_size(w, x):
 def out_proj(w, x, gate=None, out=None, workspace=None, stream=None):
     """W_o projection (attn.rs:281-285): out (M, N) = (x * sigmoid(gate)) @ W^T with
     W the Q4_K weight rows w (N, K // 256 * 144) and x, gate (M, K) float32."""
+    if stream is None and out is not None and workspace is not None:
+        rc = (_host or _load_host()).out_proj(w, x, gate, out, workspace)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return out
     M, K = x.shape
     if out is None:
         out = torch.empty((M, w.shape[0]), dtype=torch.float32, device=x.device)
@@ -383,6 +440,12 @@ def out_proj(w, x, gate=None, out=None, workspace=None, stream=None):
 
 def fill_causal_mask(mask, step_start, stream=None):
     """Device fill of the F16 mask (n_q, n_kv): row t allows keys <= step_start + t."""
+    if stream is None:
+        rc = (_host or _load_host()).fill_mask(mask, step_start)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return mask
     tm = mask_desc(mask)
     _check(lib().sqa_fill_causal_mask(ctypes.byref(tm), step_start, _stream(stream)))
     return mask
@@ -470,6 +533,10 @@ class KvCache:
 
     def append(self, slot, k_cur, v_cur, idx, stream=None):
         """Quantize this step's K/V rows, float32 (n_tokens, Hkv*D), into layer `slot`."""
+        if stream is None:
+            rc = (_host or _load_host()).append(self._h, slot, k_cur, v_cur, idx)
+            if rc is not None:
+                return _check(rc)
         n_tok, ne0 = k_cur.shape
         tk = Tensor.make(TYPE_F32, [ne0, n_tok], [4, k_cur.stride(0) * 4], k_cur.data_ptr())
         tv = Tensor.make(TYPE_F32, [ne0, n_tok], [4, v_cur.stride(0) * 4], v_cur.data_ptr())

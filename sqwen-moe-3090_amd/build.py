@@ -1,7 +1,9 @@
-"""Compile the HIP/C++ sources of this package into libsqattn.so for gfx950.
+"""Compile the HIP/C++ sources of this package into libsqattn.so for gfx950, and
+the Python binding of its hot entry points into _sqahost.so.
 
-Every source is compiled by hipcc (-x hip) into _build/, then linked into a
-shared library next to this file. Flags:
+Every source of csrc/ is compiled by hipcc (-x hip) into _build/, then linked
+into a shared library next to this file; binding/host.cpp is host code against
+torch's C++ headers. Flags:
   -Xclang -target-feature -Xclang -packed-fp32-ops   no packed fp32 VALU ops
   -ffp-contract=fast-honor-pragmas is hipcc's default; code that must round
   every multiply and add on its own (the q4_0 quantizer, the K/Q producer)
@@ -13,10 +15,12 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libsqattn.so")
+HOST = os.path.join(HERE, "_sqahost.so")
 ARCH = os.environ.get("SQA_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -51,21 +55,44 @@ def _compile(src, out):
     return out
 
 
+def _run(cmd, what):
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n" + r.stderr)
+
+
+def _compile_host(out):
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")]
+    _run([HIPCC, "-std=c++17", "-O2", "-fPIC", "-Wall", "-x", "c++", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+         + [f"-isystem{i}" for i in inc]
+         + ["-c", os.path.join(HERE, "binding", "host.cpp"), "-o", out], "hipcc of binding/host.cpp")
+    return [f"-L{os.path.join(root, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose=False):
     bdir = os.path.join(HERE, "_build")
     os.makedirs(bdir, exist_ok=True)
     srcs = sources()
     outs = [os.path.join(bdir, os.path.basename(s) + ".o") for s in srcs]
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    host = os.path.join(bdir, "host.o")
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host_libs = ex.submit(_compile_host, host)
         list(ex.map(_compile, srcs, outs))
+        host_libs = host_libs.result()
     tmp = LIB + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + outs
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError("link failed:\n" + r.stderr)
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + outs, "link")
     os.replace(tmp, LIB)
+    # finds libsqattn.so beside itself; torch's libraries are loaded with torch
+    tmp = HOST + ".tmp"
+    _run([HIPCC, "-shared", "-fPIC", "-o", tmp, host, f"-L{HERE}", "-l:libsqattn.so", "-Wl,-rpath,$ORIGIN"] + host_libs,
+         "link of the binding")
+    os.replace(tmp, HOST)
     if verbose:
-        print("built", LIB)
+        print("built", LIB, HOST)
     return LIB
 
 
