@@ -18,7 +18,7 @@
 //         (x0*c - x1*s, x0*s + x1*c); dims >= n_rot pass through;
 //   q4_0: ggml's quantize_row_q4_0_ref (q4_0_block.hpp).
 //
-// Layout: one workgroup per token. Its first n_rot/2 threads form the token's
+// Layout: one workgroup per token and group of heads (launch_d). Its first n_rot/2 threads form the token's
 // cos/sin table in LDS (as ggml forms one cache per token), then the heads stream
 // through D/4 lanes per head row, 4 consecutive dims each, so the 8 lanes of a
 // 32-value block hold it as the quantizer wants. The rotation partner of dim d
@@ -29,6 +29,7 @@ namespace sqa {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kGroups = 4;  // workgroups per CU up to which heads are split
 
 struct ProducerParams {
     const char *src;
@@ -95,7 +96,8 @@ __global__ __launch_bounds__(kThreads) void rope_norm_kernel(ProducerParams p) {
     const int l = tid % kLanes;
     const int sh = half >> 2;  // lanes between the two dims of a pair
     const int lp = 4 * l < half ? l + sh : (4 * l < p.n_rot ? l - sh : l);
-    for (int h = tid / kLanes; h < p.n_head; h += kRowsPerPass) {  // uniform per row group
+    // uniform per row group
+    for (int h = blockIdx.y * kRowsPerPass + tid / kLanes; h < p.n_head; h += gridDim.y * kRowsPerPass) {
         const float *x = reinterpret_cast<const float *>(p.src + h * p.src_nb1 + t * p.src_nb2) + 4 * l;
         float v[4];
         if constexpr (kVec) {
@@ -153,11 +155,18 @@ __global__ __launch_bounds__(kThreads) void rope_norm_kernel(ProducerParams p) {
 
 template <int D, bool kQ4>
 void launch_d(const ProducerParams &p, bool vec, hipStream_t s) {
-    const int64_t grid = p.n_tok;  // one workgroup per token
+    // The heads of a token are split over workgroups, down to one pass of heads
+    // each, while that leaves at most kGroups per CU: with few tokens the passes run
+    // side by side (each forms the rotation table again) instead of one after the
+    // other: 16 heads, 1 token 6.3 -> 4.1 us, 300 tokens 7.4 -> 5.8.
+    constexpr int kRowsPerPass = kThreads / (D / 4);
+    const int64_t passes = (p.n_head + kRowsPerPass - 1) / kRowsPerPass;
+    const int64_t room = kGroups * (int64_t)device_cu_count() / p.n_tok;
+    const dim3 grid((unsigned)p.n_tok, (unsigned)(room < 1 ? 1 : (room < passes ? room : passes)));
     if (vec)
-        rope_norm_kernel<D, kQ4, true><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(p);
+        rope_norm_kernel<D, kQ4, true><<<grid, dim3(kThreads), 0, s>>>(p);
     else
-        rope_norm_kernel<D, kQ4, false><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(p);
+        rope_norm_kernel<D, kQ4, false><<<grid, dim3(kThreads), 0, s>>>(p);
 }
 
 template <bool kQ4>

@@ -136,3 +136,17 @@ def test_cache_written_by_producer_feeds_attention(sqa, orc, dev):
     got = out.cpu().numpy()
     rms = np.sqrt((want.astype(np.float64) ** 2).mean())
     assert np.abs(got - want).max() <= 2e-3 * rms
+
+
+@pytest.mark.parametrize("n_tok,n_head", [(1, 5), (1, 16), (300, 16), (600, 7), (1100, 9)])
+def test_heads_over_workgroups(sqa, dev, n_tok, n_head):
+    """The split of a token's heads over workgroups (all passes side by side, some,
+    none) changes no value: equal to one call per head."""
+    src = torch.randn((n_tok, n_head, 256), device=dev)
+    w = torch.rand(256, device=dev)
+    pos = torch.arange(4 * n_tok, dtype=torch.int32, device=dev) * 31
+    rope = sqa.rope_params(64, (11, 11, 10, 0), 1e7)
+    got = sqa.rope_norm_f32(torch.zeros_like(src), src, w, 1e-6, pos, rope)
+    for h in range(n_head):
+        one = src[:, h:h + 1].contiguous()
+        assert torch.equal(got[:, h:h + 1], sqa.rope_norm_f32(torch.zeros_like(one), one, w, 1e-6, pos, rope))
