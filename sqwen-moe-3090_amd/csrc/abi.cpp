@@ -164,19 +164,9 @@ int sqa_supports_set_rows(const sqa_tensor *dst, const sqa_tensor *src, const sq
 
 int sqa_set_rows_q4_0(const sqa_tensor *dst, const sqa_tensor *src, const sqa_tensor *idx,
                       void *stream) {
-    if (!dst || !src || !idx) return set_error(SQA_ERR_INVALID, "set_rows: null tensor");
-    if (src->ne[1] > 0 && (!dst->data || !src->data || !idx->data))
-        return set_error(SQA_ERR_INVALID, "set_rows: null data pointer");
-    if (dst->type != SQA_TYPE_Q4_0 || src->type != SQA_TYPE_F32 || idx->type != SQA_TYPE_I64)
-        return set_error(SQA_ERR_INVALID, "set_rows: types must be q4_0 <- F32 at I64");
-    if (src->ne[0] != dst->ne[0] || idx->ne[0] != src->ne[1])
-        return set_error(SQA_ERR_INVALID, "set_rows: shape mismatch");
-    if (src->ne[0] % SQA_QK4_0)
-        return set_error(SQA_ERR_INVALID, "set_rows: row length %lld not a multiple of 32",
-                         (long long)src->ne[0]);
-    if (!sqa_supports_set_rows(dst, src, idx))
-        return set_error(SQA_ERR_UNSUPPORTED, "set_rows: strides/alignment not supported");
-    return launch_set_rows_q4_0(*dst, *src, *idx, (hipStream_t)stream);
+    const int rc = check_set_rows(dst, src, idx);
+    if (rc != SQA_OK) return rc;
+    return launch_set_rows_q4_0(*dst, *src, nullptr, nullptr, *idx, (hipStream_t)stream);
 }
 
 // ---- K/Q producer: norm + IMROPE (+ q4_0 set_rows) ----------------------------
@@ -420,3 +410,19 @@ int sqa_fill_causal_mask(const sqa_tensor *mask, int64_t step_start, void *strea
 }
 
 }  // extern "C"
+
+int sqa::check_set_rows(const sqa_tensor *dst, const sqa_tensor *src, const sqa_tensor *idx) {
+    if (!dst || !src || !idx) return set_error(SQA_ERR_INVALID, "set_rows: null tensor");
+    if (src->ne[1] > 0 && (!dst->data || !src->data || !idx->data))
+        return set_error(SQA_ERR_INVALID, "set_rows: null data pointer");
+    if (dst->type != SQA_TYPE_Q4_0 || src->type != SQA_TYPE_F32 || idx->type != SQA_TYPE_I64)
+        return set_error(SQA_ERR_INVALID, "set_rows: types must be q4_0 <- F32 at I64");
+    if (src->ne[0] != dst->ne[0] || idx->ne[0] != src->ne[1])
+        return set_error(SQA_ERR_INVALID, "set_rows: shape mismatch");
+    if (src->ne[0] % SQA_QK4_0)
+        return set_error(SQA_ERR_INVALID, "set_rows: row length %lld not a multiple of 32",
+                         (long long)src->ne[0]);
+    if (!sqa_supports_set_rows(dst, src, idx))
+        return set_error(SQA_ERR_UNSUPPORTED, "set_rows: strides/alignment not supported");
+    return SQA_OK;
+}

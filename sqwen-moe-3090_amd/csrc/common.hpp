@@ -37,8 +37,11 @@ int profile_start(const char *name, hipStream_t s);
 void profile_stop(int slot, hipStream_t s);
 
 // Kernel launchers (defined next to their kernels).
-int launch_set_rows_q4_0(const sqa_tensor &dst, const sqa_tensor &src, const sqa_tensor &idx,
-                         hipStream_t s);
+// dst2, src2: a second write of the same shape and rows in the same launch, or null
+int launch_set_rows_q4_0(const sqa_tensor &dst, const sqa_tensor &src, const sqa_tensor *dst2, const sqa_tensor *src2,
+                         const sqa_tensor &idx, hipStream_t s);
+// sqa_set_rows_q4_0's checks (abi.cpp)
+int check_set_rows(const sqa_tensor *dst, const sqa_tensor *src, const sqa_tensor *idx);
 // Norm + IMROPE producer; idx != null: q4_0 quantize-on-write into dst rows,
 // else F32 output (rope_norm_q4_0.hip). theta_scale = powf(freq_base, -2/n_rot).
 int launch_rope_norm(const sqa_tensor *dst, const sqa_tensor &src, const sqa_tensor *norm_w, float eps,

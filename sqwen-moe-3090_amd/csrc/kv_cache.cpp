@@ -170,10 +170,12 @@ int sqa_kv_cache_append(sqa_kv_cache *kv, int32_t slot, const sqa_tensor *k_cur,
     dst.nb[1] = (uint64_t)rg;
     dst.nb[2] = dst.nb[3] = (uint64_t)(rg * kv->kv_cap_alloc);
     dst.data = kv->k[slot];
-    int rc = sqa_set_rows_q4_0(&dst, k_cur, idx, stream);
+    sqa_tensor dst_v = dst;
+    dst_v.data = kv->v[slot];
+    int rc = check_set_rows(&dst, k_cur, idx);
+    if (!rc) rc = check_set_rows(&dst_v, v_cur, idx);
     if (rc) return rc;
-    dst.data = kv->v[slot];
-    return sqa_set_rows_q4_0(&dst, v_cur, idx, stream);
+    return launch_set_rows_q4_0(dst, *k_cur, &dst_v, v_cur, *idx, (hipStream_t)stream);
 }
 
 }  // extern "C"

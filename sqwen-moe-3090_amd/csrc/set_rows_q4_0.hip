@@ -13,11 +13,20 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// blockIdx.y picks one of up to two writes of the same shape (a step's K and V
+// rows): one launch of both where two took 3 us each for 512 rows, and the
+// second's gap.
+struct SetRows {
+    uint8_t *dst;
+    int64_t dst_nb1, dst_rows;
+    const char *src;
+    int64_t src_nb1;
+};
+
 template <bool kVec>
-__global__ __launch_bounds__(kThreads) void set_rows_q4_0_kernel(
-    uint8_t *__restrict__ dst, int64_t dst_nb1, int64_t dst_rows, const char *__restrict__ src,
-    int64_t src_nb1, const char *__restrict__ idx, int64_t idx_nb0, int64_t n_rows,
-    int blocks_per_row) {
+__global__ __launch_bounds__(kThreads) void set_rows_q4_0_kernel(SetRows k, SetRows v, const char *__restrict__ idx,
+                                                                 int64_t idx_nb0, int64_t n_rows, int blocks_per_row) {
+    const SetRows &p = blockIdx.y ? v : k;
     const int64_t gid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     const int64_t blk = gid >> 3;
     const int t = threadIdx.x & 7;
@@ -25,41 +34,42 @@ __global__ __launch_bounds__(kThreads) void set_rows_q4_0_kernel(
     const int64_t row = blk / blocks_per_row;
     const int b = (int)(blk - row * blocks_per_row);
     const int64_t r = *reinterpret_cast<const int64_t *>(idx + row * idx_nb0);
-    if (r < 0 || r >= dst_rows) return;  // same row for all 8 lanes of the group
+    if (r < 0 || r >= p.dst_rows) return;  // same row for all 8 lanes of the group
 
-    const float *x = reinterpret_cast<const float *>(src + row * src_nb1) + b * SQA_QK4_0 + 4 * t;
-    float v[4];
+    const float *x = reinterpret_cast<const float *>(p.src + row * p.src_nb1) + b * SQA_QK4_0 + 4 * t;
+    float f[4];
     if constexpr (kVec) {
-        const float4 f = *reinterpret_cast<const float4 *>(x);
-        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        const float4 q = *reinterpret_cast<const float4 *>(x);
+        f[0] = q.x; f[1] = q.y; f[2] = q.z; f[3] = q.w;
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = x[j];
+        for (int j = 0; j < 4; ++j) f[j] = x[j];
     }
 
-    quantize_q4_0_block8(v, t, dst + r * dst_nb1 + (int64_t)b * SQA_Q4_0_BLOCK_BYTES);
+    quantize_q4_0_block8(f, t, p.dst + r * p.dst_nb1 + (int64_t)b * SQA_Q4_0_BLOCK_BYTES);
 }
 
 }  // namespace
 
-int launch_set_rows_q4_0(const sqa_tensor &dst, const sqa_tensor &src, const sqa_tensor &idx,
-                         hipStream_t s) {
+int launch_set_rows_q4_0(const sqa_tensor &dst, const sqa_tensor &src, const sqa_tensor *dst2, const sqa_tensor *src2,
+                         const sqa_tensor &idx, hipStream_t s) {
     const int64_t n_rows = src.ne[1];
     const int bpr = (int)(src.ne[0] / SQA_QK4_0);
     if (n_rows == 0) return SQA_OK;
     const int64_t total_lanes = n_rows * bpr * 8;
-    const int64_t grid = (total_lanes + kThreads - 1) / kThreads;
-    const bool vec = ((uintptr_t)src.data % 16 == 0) && (src.nb[1] % 16 == 0);
+    const dim3 grid((unsigned)((total_lanes + kThreads - 1) / kThreads), dst2 ? 2 : 1);
+    auto of = [](const sqa_tensor &d, const sqa_tensor &x) {
+        return SetRows{(uint8_t *)d.data, (int64_t)d.nb[1], d.ne[1], (const char *)x.data, (int64_t)x.nb[1]};
+    };
+    auto vec16 = [](const sqa_tensor &x) { return (uintptr_t)x.data % 16 == 0 && x.nb[1] % 16 == 0; };
+    const SetRows k = of(dst, src), v = dst2 ? of(*dst2, *src2) : k;
     const int prof = profile_start("set_rows_q4_0", s);
-    if (vec) {
-        set_rows_q4_0_kernel<true><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(
-            (uint8_t *)dst.data, (int64_t)dst.nb[1], dst.ne[1], (const char *)src.data,
-            (int64_t)src.nb[1], (const char *)idx.data, (int64_t)idx.nb[0], n_rows, bpr);
-    } else {
-        set_rows_q4_0_kernel<false><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(
-            (uint8_t *)dst.data, (int64_t)dst.nb[1], dst.ne[1], (const char *)src.data,
-            (int64_t)src.nb[1], (const char *)idx.data, (int64_t)idx.nb[0], n_rows, bpr);
-    }
+    if (vec16(src) && (!src2 || vec16(*src2)))
+        set_rows_q4_0_kernel<true><<<grid, dim3(kThreads), 0, s>>>(k, v, (const char *)idx.data, (int64_t)idx.nb[0],
+                                                                   n_rows, bpr);
+    else
+        set_rows_q4_0_kernel<false><<<grid, dim3(kThreads), 0, s>>>(k, v, (const char *)idx.data, (int64_t)idx.nb[0],
+                                                                    n_rows, bpr);
     profile_stop(prof, s);
     return hip_status(hipGetLastError(), "set_rows_q4_0 launch");
 }

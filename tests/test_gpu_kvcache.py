@@ -170,3 +170,20 @@ def test_graph_replayed_decode_step_matches_oracle(sqa, orc, dev):
         g.replay()
         torch.cuda.synchronize()
         _check_layer(kv, orc, 0, q, mask, out, k_cur, v_cur, s0, f"graph replay {r}")
+
+
+@pytest.mark.parametrize("n_tok,off_k,off_v", [(1, 0, 0), (5, 1, 0), (7, 0, 3), (300, 1, 1)])
+def test_append_of_unaligned_rows(sqa, dev, n_tok, off_k, off_v):
+    """One launch writes K and V: rows off a 16-byte boundary on either side give
+    the bytes of two single writes."""
+    W = 512
+    src = [torch.randn(n_tok * W + 4, device=dev)[o:o + n_tok * W].view(n_tok, W) for o in (off_k, off_v)]
+    idx = torch.randperm(n_tok, device=dev)
+    kv = sqa.KvCache(1, 256, 2, 512)
+    kv.zero_caches()
+    kv.begin_step(n_tok)
+    kv.append(0, *src, idx)
+    for got, x in zip((kv.k[0], kv.v[0]), src):
+        want = torch.zeros_like(got)
+        sqa.set_rows_q4_0(want, x.clone(), idx)
+        assert torch.equal(got, want) and bool(got[:n_tok].any())
