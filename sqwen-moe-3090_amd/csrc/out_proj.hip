@@ -11,20 +11,14 @@
 // 64j + 32 + l in the high one). A value is d*scale*code - dmin*min.
 //
 // Up to 4 tokens (decode, verify) one kernel, op_gemv (below); more tokens two:
-//   op_prep  one thread per (token, 32-value sub-block): xg = x * sigmoid(gate)
-//            in fp32, written as an fp16 hi + lo pair (xg = hi + lo to ~22
-//            bits) [M16][K], plus the sub-block sum S = sum xg [M16][K/32];
-//            tokens M..M16-1 (M16 = M rounded up to 16) are zeros
-//   op_gemm  16x16x32 f16 MFMAs over the raw codes: per sub-block the A operand
-//            is the 4-bit codes as fp16 subnormals (code * 2^-24 for low
-//            nibbles, code * 2^-20 for high ones: exact, one v_perm and one
-//            v_and per two codes), B = xg hi and lo, so C = sum code * xg has
-//            every product exact; the wave then adds (d*scale*2^24 or 2^20) * C
-//            - dmin*min * S per (row, token). Rows of W are read once per token
-//            tile straight from the weight bytes.
-// A workgroup owns 16 rows (decode: 16 wavefronts) or 64 rows (4 wavefronts)
-// and one tile of 16 tokens; its wavefronts split K by super-block and add
-// their partial sums through LDS.
+//   op_prep   xg = x * sigmoid(gate) in fp32, written as an fp16 hi + lo pair (xg
+//             = hi + lo to ~22 bits) in the order of the MFMA's B operand, and
+//             the sub-block sums S = sum xg as the B operand of the min term
+//   op_gemm   16x16x32 f16 MFMAs over the raw codes: every product exact, then d
+//             and dmin per super-block in fp32. Two forms by the amount of work:
+//             op_gemm (K split over the wavefronts, no barrier) while its tiles
+//             give a CU at most one workgroup, else op_gemm2 (operands shared
+//             through LDS)
 //
 // MFMA operand layouts (lane = 16*g + n):
 //   16x16x32 f16: A[n][8g..8g+7]   B[8g..8g+7][n]   C[4g..4g+3][n]
@@ -37,10 +31,10 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kQK = 256;           // values per Q4_K super-block
 constexpr int kBlockBytes = 144;   // bytes per super-block
-constexpr int kSubs = kQK / 32;    // sub-blocks per super-block
 constexpr int kGemvTokens = 4;     // token counts up to this take op_gemv
 
 __device__ __forceinline__ float h2f(uint32_t bits) {
@@ -51,286 +45,330 @@ __device__ __forceinline__ float h2f(uint32_t bits) {
 }
 
 // ---------------------------------------------------------------- op_prep
-// One thread per 8 values (a quarter sub-block) of one token: xg = x *
-// sigmoid(gate) as an fp16 hi + lo pair, and through the lane quad the
-// sub-block sum S (f32) and its hi + lo slots for the min MFMA of op_gemm2.
-// Tokens M..Mp-1 and the sub-blocks that pad K to whole groups of four
-// super-blocks are zeros. x (and gate) rows are 16-byte aligned when VEC.
+// One wavefront per (16 tokens, 64 values of K): lane 16q + n takes values 8q ..
+// 8q + 7 of both 32-value sub-blocks of token n and writes xg = x *
+// sigmoid(gate) as fp16 hi and lo in the order in which op_gemm reads them, 1 KB
+// per load. B operand (c, e) of super-block s, c < 4, e < 2, holds in lane 16g + n
+// the values 64g + 32e + 8c .. + 7 of token n: an MFMA then takes from each lane
+// group another code group (64 values, 32 bytes of a weight row), so a lane needs
+// 32 consecutive weight bytes and two of the 8 scales. hi and lo of tile T at
+// ((T * K/256 + s) * 8 + 2c + e) * 2 KB. The sub-block sums S go out as three bf16
+// parts each (24 bits, fp32's range): the B operand of the min MFMA of
+// super-block s, 1 KB at (T * K/256 + s), where lane 16g + n holds S of sub-blocks
+// 2g, 2g + 1 as {s0, s1} of part 0, of part 1, of part 2, and two zeros. Tokens
+// M.. of the last tile are zeros. x (and gate) rows are 16-byte aligned when VEC.
+__device__ __forceinline__ float xsum16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float xsum32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 template <bool GATE, bool VEC>
 __global__ __launch_bounds__(256) void op_prep_kernel(const char *__restrict__ x, int64_t x_nb1,
                                                       const char *__restrict__ gate, int64_t g_nb1, int K, int M,
-                                                      int Mp, int nq, uint16_t *__restrict__ xh,
-                                                      uint16_t *__restrict__ xl, float *__restrict__ S,
-                                                      uint16_t *__restrict__ sp) {
-    const int subs = K / 32, psubs = 32 * nq;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)Mp * psubs * 4) return;  // whole quads: the total is a multiple of 4
-    const int qtr = (int)(idx & 3);
-    const int64_t ts = idx >> 2;
-    const int t = (int)(ts / psubs), s = (int)(ts - (int64_t)t * psubs);
-    float v[8], gv[8];
+                                                      int tiles, uint4 *__restrict__ xb, uint4 *__restrict__ sb) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int kp = K / 64;  // sub-block pairs
+    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wid >= (int64_t)tiles * kp) return;
+    const int T = (int)(wid / kp), pr = (int)(wid - (int64_t)T * kp);
+    const int t = 16 * T + n;
+    uint32_t sw[2][3];  // the three parts of S of both sub-blocks
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
-    if (t < M && s < subs) {
-        const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 32 * s + 8 * qtr;
-        const float *gr = GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 32 * s + 8 * qtr : nullptr;
-        if (VEC) {
+    for (int e = 0; e < 2; ++e) {
+        float v[8], gv[8];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                const float4 a = reinterpret_cast<const float4 *>(xr)[c];
-                v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
-                if (GATE) {
-                    const float4 b = reinterpret_cast<const float4 *>(gr)[c];
-                    gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
+        for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
+        if (t < M) {
+            const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 64 * pr + 32 * e + 8 * g;
+            const float *gr =
+                GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 64 * pr + 32 * e + 8 * g : nullptr;
+            if (VEC) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const float4 a = reinterpret_cast<const float4 *>(xr)[c];
+                    v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
+                    if (GATE) {
+                        const float4 b = reinterpret_cast<const float4 *>(gr)[c];
+                        gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    v[j] = xr[j];
+                    if (GATE) gv[j] = gr[j];
                 }
             }
-        } else {
+            if (GATE) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                v[j] = xr[j];
-                if (GATE) gv[j] = gr[j];
+                for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
             }
         }
-        if (GATE) {
+        float sum = 0.0f;
+        uint16_t hb[8], lb[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
+        for (int j = 0; j < 8; ++j) {
+            sum += v[j];
+            float a = v[j];
+            // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
+            asm volatile("" : "+v"(a));
+            const _Float16 h = (_Float16)a;
+            const _Float16 l = (_Float16)(a - (float)h);
+            __builtin_memcpy(&hb[j], &h, 2);
+            __builtin_memcpy(&lb[j], &l, 2);
+        }
+        uint4 a, b;
+        __builtin_memcpy(&a, hb, 16);
+        __builtin_memcpy(&b, lb, 16);
+        uint4 *o = xb + ((int64_t)T * (2 * kp) + 8 * (pr >> 2) + 2 * g + e) * 128 + 16 * (pr & 3) + n;
+        o[0] = a;
+        o[64] = b;
+        // S = its leading 8 bits (truncated) + those of the rest, twice: each
+        // difference is exact
+        float r = xsum32(xsum16(sum));
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const uint32_t top = __float_as_uint(r) & 0xFFFF0000u;
+            sw[e][c] = top >> 16;
+            r -= __uint_as_float(top);
         }
     }
-    float sum = 0.0f;
-    uint16_t hb[8], lb[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        sum += v[j];
-        float a = v[j];
-        // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
-        asm volatile("" : "+v"(a));
-        const _Float16 h = (_Float16)a;
-        const _Float16 l = (_Float16)(a - (float)h);
-        __builtin_memcpy(&hb[j], &h, 2);
-        __builtin_memcpy(&lb[j], &l, 2);
-    }
-    // sum over the quad (quad_perm [1,0,3,2], then [2,3,0,1])
-    sum += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum), 0xB1, 0xf, 0xf, false));
-    sum += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum), 0x4E, 0xf, 0xf, false));
-    if (qtr == 0) {
-        // S hi + lo in the slot order of the min MFMA: group q of 4 super-blocks,
-        // slot 8g + e = sub-block 2g + (e & 1) of super-block 4q + (e >> 1)
-        const int sb = s >> 3, sub = s & 7;
-        const int slot = 8 * (sub >> 1) + 2 * (sb & 3) + (sub & 1);
-        float a = sum;
-        asm volatile("" : "+v"(a));
-        const _Float16 h = (_Float16)a;
-        const _Float16 l = (_Float16)(a - (float)h);
-        uint16_t *o = sp + ((int64_t)t * nq + (sb >> 2)) * 64 + slot;
-        __builtin_memcpy(o, &h, 2);
-        __builtin_memcpy(o + 32, &l, 2);
-        if (s < subs) S[(int64_t)t * subs + s] = sum;  // [token][sub-block]
-    }
-    if (s >= subs) return;
-    uint4 a, b;
-    __builtin_memcpy(&a, hb, 16);
-    __builtin_memcpy(&b, lb, 16);
-    *reinterpret_cast<uint4 *>(xh + (int64_t)t * K + 32 * s + 8 * qtr) = a;
-    *reinterpret_cast<uint4 *>(xl + (int64_t)t * K + 32 * s + 8 * qtr) = b;
+    if (g == (pr & 3))
+        sb[((int64_t)T * (kp / 4) + (pr >> 2)) * 64 + lane] =
+            make_uint4(sw[0][0] | (sw[1][0] << 16), sw[0][1] | (sw[1][1] << 16), sw[0][2] | (sw[1][2] << 16), 0u);
 }
 
 // ---------------------------------------------------------------- op_gemm
+// What a lane (g, n) keeps of the super-block header of row n: scales and mins of
+// sub-blocks 2g and 2g + 1 (ggml's get_scale_min_k4, branch-free: sub-blocks 0-3
+// have 6 bits in bytes s and s + 4 of the 12, 4-7 four bits in byte s + 4 and two
+// on top of bytes s - 4 and s), and d | dmin of the row.
+struct OpHead {
+    uint32_t sc0, sc1, mins, d;
+};
+__device__ __forceinline__ OpHead op_head(uint4 hd, int g) {
+    const uint32_t sh = 16u * (uint32_t)(g & 1);
+    const uint32_t q0 = hd.y >> sh, q1 = hd.z >> sh, q2 = hd.w >> sh;  // bytes of 2g, 2g + 1 (mod 4)
+    const bool top = g >= 2;
+    const uint32_t sc = top ? (q2 & 0x0F0Fu) | ((q0 >> 2) & 0x3030u) : q0 & 0x3F3Fu;
+    const uint32_t mn = top ? ((q2 >> 4) & 0x0F0Fu) | ((q1 >> 2) & 0x3030u) : q1 & 0x3F3Fu;
+    OpHead h;
+    h.sc0 = sc & 0xFFu;
+    h.sc1 = sc >> 8;
+    // bf16 of the integers: their fp32 bits end in zeros
+    h.mins = (__float_as_uint((float)(mn & 0xFFu)) >> 16) | (__float_as_uint((float)(mn >> 8)) & 0xFFFF0000u);
+    h.d = hd.x;
+    return h;
+}
+
+// A operands of a step: 8 code bytes, low nibbles (sub-block 2g) and high (2g + 1)
+// as code * scale * 2^-24 (see op_gemm)
+__device__ __forceinline__ void op_a_operand(const OpHead &h, uint32_t qx, uint32_t qy, half8 &alo, half8 &ahi) {
+    uint32_t sp[4];  // bytes 2m, 2m+1 spread to the two halves of dword m
+    sp[0] = __builtin_amdgcn_perm(0u, qx, 0x0c010c00u);
+    sp[1] = __builtin_amdgcn_perm(0u, qx, 0x0c030c02u);
+    sp[2] = __builtin_amdgcn_perm(0u, qy, 0x0c010c00u);
+    sp[3] = __builtin_amdgcn_perm(0u, qy, 0x0c030c02u);
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        lo[m] = __umul24(sp[m] & 0x000F000Fu, h.sc0);
+        hi[m] = __umul24((sp[m] >> 4) & 0x000F000Fu, h.sc1);
+    }
+    __builtin_memcpy(&alo, lo, 16);
+    __builtin_memcpy(&ahi, hi, 16);
+}
+
+// acc += d 2^24 C - dmin * (mins . S) of one super-block and row tile
+template <int TT>
+__device__ __forceinline__ void op_scale_add(const OpHead &h, int g, const floatx4 (&C)[TT], const uint4 (&sv)[TT],
+                                             floatx4 (&acc)[TT]) {
+    const uint32_t aw[4] = {h.mins, h.mins, h.mins, 0u};
+    bf16x8 am;
+    __builtin_memcpy(&am, aw, 16);
+    float d[4], dm[4];  // d 2^24 and dmin of C rows 4g..4g+3
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t w = (uint32_t)__shfl((int)h.d, 4 * g + i);
+        d[i] = h2f(w & 0xffffu) * 16777216.0f;
+        dm[i] = h2f(w >> 16);
+    }
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        bf16x8 bm;
+        __builtin_memcpy(&bm, &sv[tt], 16);
+        const floatx4 cm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[tt][i] = fmaf(-dm[i], cm[i], fmaf(d[i], C[tt][i], acc[tt][i]));
+    }
+}
+
+// Workgroups go round-robin to the 8 XCDs: the id of workgroup lin such that each
+// XCD takes a contiguous run of ids, i.e. of token tiles (every row block of
+// them), and its L2 serves their operands to all their row blocks.
+__device__ __forceinline__ int xcd_order(int lin, int nb) {
+    const int x = lin & 7, per = nb >> 3, rem = nb & 7;
+    return x * per + (x < rem ? x : rem) + (lin >> 3);
+}
+
 struct GemmParams {
     const uint8_t *w;
     int64_t w_nb1;
-    const uint16_t *xh, *xl;
-    const float *S;
-    int K, N, M, M16;
+    const uint4 *xb, *sb;  // B operands, see op_prep
+    int K, N, M, tiles;    // tiles of 16 tokens
+    int row_blocks;        // workgroups along N
     float *dst;
     int64_t d_nb1;
 };
 
-// (scale, min) of sub-block s from the 12 scale bytes b[0..11], held as three
-// dwords q0 = b[0..3], q1 = b[4..7], q2 = b[8..11]
-__device__ __forceinline__ void scale_min(uint32_t q0, uint32_t q1, uint32_t q2, int s, int &sc, int &mn) {
-    if (s < 4) {
-        sc = (q0 >> (8 * s)) & 63;
-        mn = (q1 >> (8 * s)) & 63;
-    } else {
-        const int r = 8 * (s - 4);
-        sc = ((q2 >> r) & 15) | (((q0 >> (r + 6)) & 3) << 4);
-        mn = ((q2 >> (r + 4)) & 15) | (((q1 >> (r + 6)) & 3) << 4);
-    }
-}
-
-// A workgroup of KS wavefronts owns 16*RT rows of W and one tile of 16 tokens;
-// wavefront w takes super-blocks w, w + KS, ... of K, and the KS partial sums
-// meet in LDS at the end. Each wavefront loads all operands of a super-block
-// (scales, codes, activations) before it computes on them.
-template <int KS, int RT>
+// A workgroup of KS wavefronts owns 16 RT rows of W and 16 TT tokens; wavefront w
+// takes super-blocks w, w + KS, ... of K, reading weights and operands straight
+// from memory (no barrier in the loop), and the KS partial sums meet in LDS.
+//   * The A operand is code * scale of the code's sub-block as an fp16 subnormal: an
+//     integer of at most 15 * 63 = 945, i.e. exactly code * scale * 2^-24 (one
+//     v_mul_u32_u24 scales the two codes of a dword, as the halves cannot carry
+//     into each other). The super-block accumulates into one MFMA chain C = 2^-24
+//     sum_k scale * code * x against x hi and lo, and acc += d 2^24 C once per
+//     super-block.
+//   * The min term is one bf16 MFMA per super-block: A = the mins (integers up to
+//     63, exact) of sub-blocks 2g, 2g + 1 three times over, B = the three parts
+//     of their S; acc -= dmin * its sum.
+// What bounds it is traffic into the CUs, (N / 16 RT) * M * K * 4 bytes of
+// operands at 64 bytes a clock and CU, and the VALU that builds A, paid once per
+// TT token tiles.
+template <int KS, int RT, int TT>
 __global__ __launch_bounds__(64 * KS) void op_gemm_kernel(GemmParams p) {
-    __shared__ float sc_lds[KS][RT][kSubs][2][16];  // per wave: scaled d*scale and dmin*min per sub-block, row
-    __shared__ float red[KS][RT][4][64];
+    __shared__ float red[KS][RT * TT][4][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int r0 = blockIdx.x * 16 * RT;
-    const int t0 = blockIdx.y * 16;
+    const int id = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int r0 = (id % p.row_blocks) * 16 * RT;
+    const int T0 = (id / p.row_blocks) * TT;
     const int nsb = p.K / kQK;
 
-    floatx4 acc[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[rt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // a column past the M tokens reads token t0's data (one broadcast row for
-    // decode) and masks it to zero
-    const int tok = t0 + n < p.M ? t0 + n : t0;
-    const uint32_t tok_mask = t0 + n < p.M ? 0xFFFFFFFFu : 0u;
-    const uint16_t *xh_t = p.xh + (int64_t)tok * p.K + 8 * g;
-    const uint16_t *xl_t = p.xl + (int64_t)tok * p.K + 8 * g;
-    const float *srow = p.S + (int64_t)tok * (p.K / 32);
-    float(*my_sc)[kSubs][2][16] = sc_lds[wave];
-    const uint8_t *wrow[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) wrow[rt] = p.w + (int64_t)(r0 + 16 * rt + n) * p.w_nb1;
-
-    for (int sb = wave; sb < nsb; sb += KS) {
-        // ---- every load of the super-block first ----
-        uint4 hdr[RT];  // d, dmin, scales[0..11] of row tile-row n
-        uint2 q[RT][4];  // codes 8g..8g+7 of both sub-blocks of group j
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const uint8_t *blk = wrow[rt] + (int64_t)sb * kBlockBytes;
-            hdr[rt] = *reinterpret_cast<const uint4 *>(blk);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) q[rt][j] = *reinterpret_cast<const uint2 *>(blk + 16 + 32 * j + 8 * g);
-        }
-        uint4 xb[4][4];  // [j][hi lo, hi lo of the high sub-block]; zeros past the M tokens
-        float sv[8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k0 = sb * kQK + 64 * j;
-            xb[j][0] = *reinterpret_cast<const uint4 *>(xh_t + k0);
-            xb[j][1] = *reinterpret_cast<const uint4 *>(xl_t + k0);
-            xb[j][2] = *reinterpret_cast<const uint4 *>(xh_t + k0 + 32);
-            xb[j][3] = *reinterpret_cast<const uint4 *>(xl_t + k0 + 32);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                xb[j][c].x &= tok_mask, xb[j][c].y &= tok_mask, xb[j][c].z &= tok_mask, xb[j][c].w &= tok_mask;
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sv[e] = __uint_as_float(__float_as_uint(srow[sb * kSubs + e]) & tok_mask);
-        // ---- scales of the wave's rows: lane (g, n) decodes sub-blocks 2g, 2g+1 of
-        // tile-row n of every row tile and publishes them by row (the LDS accesses
-        // of one wavefront complete in order: no barrier) ----
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const float d = h2f(hdr[rt].x & 0xffffu), dmin = h2f(hdr[rt].x >> 16);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int s = 2 * g + e;
-                int sc, mn;
-                scale_min(hdr[rt].y, hdr[rt].z, hdr[rt].w, s, sc, mn);
-                // even sub-blocks read low nibbles (code * 2^-24), odd ones high (2^-20)
-                my_sc[rt][s][0][n] = d * (float)sc * (e == 0 ? 16777216.0f : 1048576.0f);
-                my_sc[rt][s][1][n] = dmin * (float)mn;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            half8 bh0, bl0, bh1, bl1;
-            __builtin_memcpy(&bh0, &xb[j][0], 16);
-            __builtin_memcpy(&bl0, &xb[j][1], 16);
-            __builtin_memcpy(&bh1, &xb[j][2], 16);
-            __builtin_memcpy(&bl1, &xb[j][3], 16);
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                uint32_t sp[4];  // bytes 2m, 2m+1 spread to the two halves of dword m
-                sp[0] = __builtin_amdgcn_perm(0u, q[rt][j].x, 0x0c010c00u);
-                sp[1] = __builtin_amdgcn_perm(0u, q[rt][j].x, 0x0c030c02u);
-                sp[2] = __builtin_amdgcn_perm(0u, q[rt][j].y, 0x0c010c00u);
-                sp[3] = __builtin_amdgcn_perm(0u, q[rt][j].y, 0x0c030c02u);
-                uint32_t lo[4], hi[4];
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    lo[m] = sp[m] & 0x000F000Fu;
-                    hi[m] = sp[m] & 0x00F000F0u;
-                }
-                half8 alo, ahi;
-                __builtin_memcpy(&alo, lo, 16);
-                __builtin_memcpy(&ahi, hi, 16);
-                floatx4 cl = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bh0, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                cl = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bl0, cl, 0, 0, 0);
-                floatx4 ch = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bh1, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                ch = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bl1, ch, 0, 0, 0);
-                const floatx4 dl = *reinterpret_cast<const floatx4 *>(&my_sc[rt][2 * j][0][4 * g]);
-                const floatx4 ml = *reinterpret_cast<const floatx4 *>(&my_sc[rt][2 * j][1][4 * g]);
-                const floatx4 dh = *reinterpret_cast<const floatx4 *>(&my_sc[rt][2 * j + 1][0][4 * g]);
-                const floatx4 mh = *reinterpret_cast<const floatx4 *>(&my_sc[rt][2 * j + 1][1][4 * g]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float a = fmaf(cl[i], dl[i], acc[rt][i]);
-                    a = fmaf(-ml[i], sv[2 * j], a);
-                    a = fmaf(ch[i], dh[i], a);
-                    acc[rt][i] = fmaf(-mh[i], sv[2 * j + 1], a);
-                }
-            }
-        }
-    }
-
-    // ---- the KS partial sums through LDS ----
+    floatx4 acc[RT][TT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) red[wave][rt][i][lane] = acc[rt][i];
-    __syncthreads();
-    // wavefront w finishes row tiles w, w + KS, ...
-    const int t = t0 + n;
-    float *drow = reinterpret_cast<float *>(reinterpret_cast<char *>(p.dst) + (int64_t)t * p.d_nb1);
-    for (int rt = wave; rt < RT; rt += KS) {
+        for (int tt = 0; tt < TT; ++tt) acc[rt][tt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const uint8_t *wrow[RT];  // rows past N read the last one and are never stored
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int r = r0 + 16 * rt + n;
+        wrow[rt] = p.w + (int64_t)(r < p.N ? r : p.N - 1) * p.w_nb1;
+    }
+    const uint4 *xt[TT], *st[TT];  // token tiles past the last one read it and are never stored
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        const int T = T0 + tt < p.tiles ? T0 + tt : p.tiles - 1;
+        xt[tt] = p.xb + (int64_t)T * (p.K / 32) * 128 + lane;
+        st[tt] = p.sb + (int64_t)T * nsb * 64 + lane;
+    }
+
+    for (int s = wave; s < nsb; s += KS) {
+        OpHead hd[RT];
+        uint4 q[RT][2];  // code group g: 8 bytes per step
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const uint8_t *blk = wrow[rt] + (int64_t)s * kBlockBytes;
+            hd[rt] = op_head(*reinterpret_cast<const uint4 *>(blk), g);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) q[rt][k] = *reinterpret_cast<const uint4 *>(blk + 16 + 32 * g + 16 * k);
+        }
+        uint4 sv[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) sv[tt] = st[tt][(int64_t)s * 64];
+        floatx4 C[RT][TT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) C[rt][tt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            half8 b[TT][4];  // operands (j, 0) hi, lo, (j, 1) hi, lo
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint4 v = xt[tt][((int64_t)s * 8 + 2 * j) * 128 + 64 * c];
+                    __builtin_memcpy(&b[tt][c], &v, 16);
+                }
+            half8 a[RT][2];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const uint4 w = q[rt][j >> 1];
+                op_a_operand(hd[rt], j & 1 ? w.z : w.x, j & 1 ? w.w : w.y, a[rt][0], a[rt][1]);
+            }
+            // the four MFMAs of a C tile apart: each waits for the one before
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int tt = 0; tt < TT; ++tt)
+                        C[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[rt][c >> 1], b[tt][c], C[rt][tt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) op_scale_add<TT>(hd[rt], g, C[rt], sv, acc[rt]);
+    }
+
+    // ---- the KS partial sums through LDS; wavefront w finishes tiles w, w + KS, ...
+    if (KS > 1) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) red[wave][rt * TT + tt][i][lane] = acc[rt][tt][i];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u0 = 0; u0 < RT * TT; u0 += KS) {
+        const int u = u0 + wave;
+        if (u >= RT * TT) break;
+        const int r = r0 + 16 * (u / TT), t = 16 * (T0 + u % TT) + n;
         float o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float a = 0.0f;
 #pragma unroll
-            for (int w = 0; w < KS; ++w) a += red[w][rt][i][lane];
+            for (int w = 0; w < KS; ++w) a += red[w][u][i][lane];
             o[i] = a;
         }
-        if (t < p.M)
-            *reinterpret_cast<float4 *>(drow + r0 + 16 * rt + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
+        if (r < p.N && t < p.M)
+            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(p.dst) + (int64_t)t * p.d_nb1 + 4 * (r + 4 * g)) =
+                make_float4(o[0], o[1], o[2], o[3]);
     }
 }
 
 // ---------------------------------------------------------------- op_gemm2
-// Larger token counts: a workgroup of 8 wavefronts owns 128 rows of W
-// (wavefront w: rows 16w..16w+15) and 32 tokens (two token tiles of 16).
-//   * Per super-block and row tile, the A operand of sub-block s is code *
-//     scale_s as an fp16 subnormal: an integer of at most 15 * 63 = 945, i.e.
-//     exactly code * scale * 2^-24 (one v_mul_u32_u24 scales the two codes of a
-//     dword, as the halves cannot carry into each other). The 8 sub-blocks then
-//     accumulate into one MFMA chain C = 2^-24 sum_k scale * code * x against x
-//     hi and lo, and acc += d 2^24 C once per super-block.
-//   * The min term sum_sb dmin * sum_s min_s * S_s runs on the MFMA as well:
-//     A = dmin * min as an fp16 hi + lo pair (17 bits) against B = S hi + lo,
-//     where k slot 8g + e of a group of four super-blocks holds sub-block
-//     2g + (e & 1) of super-block 4q + (e >> 1), so that each lane fills its
-//     two slots from the super-block it already holds.
-//   * Everything comes HBM -> LDS by DMA, double buffered: half a super-block
-//     of activations (128 values x 32 tokens, hi and lo: 16 KB, chunk c of
-//     token row t at c ^ (t & 15)), the 128 weight rows' super-block (18 KB)
-//     and, one group of four super-blocks ahead, the S hi/lo slots (4 KB).
-//     Each wait counts the wavefront's younger DMAs, so the stages in flight
-//     are not waited for.
+// More tokens: a workgroup of 8 wavefronts owns 128 rows of W (wavefront w: rows
+// 16w..16w+15) and 32 tokens; the arithmetic is op_gemm's. Everything comes HBM ->
+// LDS by DMA, double buffered: the operands of half a super-block (two steps, 2
+// tiles, hi and lo: 16 KB, shared by the eight wavefronts), the 128 weight rows'
+// super-block (18 KB) and the S operands (2 KB). 512 tokens, N = 2048, K = 4096:
+// 28 us; each wavefront reads every operand, 16 KB a half and wavefront, and
+// those LDS reads (128 bytes a clock) cost more than the MFMAs they feed. Measured
+// and slower: 64 tokens a workgroup (48 us with op_prep, 33 this form: half the
+// CUs idle; equal from 1024 tokens), activations two halves ahead in three buffers
+// (34, and 64 against 55 at 1024 tokens: one workgroup per CU), 64 rows (36 at
+// 512), two row tiles per wavefront with the K halves on two sets of four
+// wavefronts and the weights straight to registers (37: the wait for the weights).
 constexpr int kG2Rows = 128;
-constexpr int kG2Tok = 32;
-constexpr int kG2RT = 1;                            // row tiles of 16 per wavefront
-constexpr int kG2Waves = kG2Rows / (16 * kG2RT);   // 8: two wavefronts per SIMD
-constexpr int kG2XInst = 16 / kG2Waves;             // activation DMA instructions per wavefront
-constexpr int kG2Half = kG2Tok * 512;        // activation bytes of half a super-block
+constexpr int kG2Waves = kG2Rows / 16;            // 8: two wavefronts per SIMD
 constexpr int kG2WBytes = kG2Rows * kBlockBytes;  // 18432
-constexpr int kG2WInst = kG2WBytes / 1024;   // 18 DMA instructions
+constexpr int kG2WInst = kG2WBytes / 1024;        // 18 DMA instructions
 constexpr int kG2WPer = (kG2WInst + kG2Waves - 1) / kG2Waves;
-constexpr int kG2SBytes = kG2Tok * 128;      // S slots of one group: [32 tokens][hi 64 B | lo 64 B]
-constexpr int kG2XAhead = 1;                  // activation halves in flight ahead of the one in use
-constexpr int kG2WAhead = 1;                  // weight super-blocks in flight ahead of the one in use
-constexpr int kG2XBufs = kG2XAhead + 1;
-constexpr int kG2WBufs = kG2WAhead + 1;
-static_assert(2 * kG2WAhead >= kG2XAhead, "a weight stage is issued no later than the activations of its first half");
-static_assert(kG2XAhead == 1, "the per-half wait drains every DMA: the activations of the next half are issued last");
+constexpr int kG2TT = 2;                          // token tiles
+constexpr int kG2Half = 4 * kG2TT * 2 * 1024;     // [step, nibble half][tile][hi, lo] of 1 KB
+constexpr int kG2XInst = kG2Half / 1024 / kG2Waves;  // activation DMA instructions per wavefront
+constexpr int kG2SBytes = kG2TT * 1024;
+// 73728 bytes of dynamic LDS: two workgroups per CU
+constexpr int kG2Lds = 2 * (kG2Half + kG2WBytes + kG2SBytes);
 static_assert(kG2WBytes % 1024 == 0, "weight stage in whole DMA instructions");
 
 // 16 bytes per lane from sbase + voff into LDS at m0 + 16 * lane, asynchronously
@@ -344,261 +382,109 @@ __device__ __forceinline__ void dma16(uint32_t voff, const void *sbase, uint32_t
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(bs), "{m0}"(ms) : "memory");
 }
 
-struct Gemm2Params {
-    const uint8_t *w;
-    int64_t w_nb1;
-    const uint16_t *x;  // xh [Mp][K]; xl starts xl_off bytes later
-    uint32_t xl_off;
-    const uint16_t *sp;  // [Mp][nq][64] fp16 S hi (32 slots) then lo (32 slots)
-    int K, N, M, Mp, nq;
-    float *dst;
-    int64_t d_nb1;
-};
-
-// 77824 bytes of dynamic LDS: two workgroups per CU (deeper rings measured slower,
-// 48 vs 36 us at 512 tokens, as they halve the workgroups a CU holds)
-constexpr int kG2Lds = kG2XBufs * kG2Half + kG2WBufs * kG2WBytes + 2 * kG2SBytes;
-
-__global__ __launch_bounds__(64 * kG2Waves) void op_gemm2_kernel(Gemm2Params p) {
+__global__ __launch_bounds__(64 * kG2Waves) void op_gemm2_kernel(GemmParams p) {
+    constexpr int TT = kG2TT;
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t(*xs)[kG2Half] = reinterpret_cast<uint8_t(*)[kG2Half]>(lds);
-    uint8_t(*wb)[kG2WBytes] = reinterpret_cast<uint8_t(*)[kG2WBytes]>(lds + kG2XBufs * kG2Half);
-    uint8_t *sb_lds = lds + kG2XBufs * kG2Half + kG2WBufs * kG2WBytes;
+    uint8_t(*wb)[kG2WBytes] = reinterpret_cast<uint8_t(*)[kG2WBytes]>(lds + 2 * kG2Half);
+    uint8_t(*ss)[kG2SBytes] = reinterpret_cast<uint8_t(*)[kG2SBytes]>(lds + 2 * (kG2Half + kG2WBytes));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    // workgroups go round-robin to the 8 XCDs: give each XCD whole token tiles
-    // (every row block of them), so an XCD's L2 serves its activations to all
-    // its row blocks
-    int bx = (int)blockIdx.x, by = (int)blockIdx.y;
-    {
-        const int nx = (int)gridDim.x, ny = (int)gridDim.y;
-        if (ny % 8 == 0) {
-            const int id = bx + nx * by, k = id / 8;
-            by = (id % 8) * (ny / 8) + k / nx;
-            bx = k % nx;
-        }
-    }
-    const int row0 = bx * kG2Rows;
-    const int t0 = by * kG2Tok;
+    const int id = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int row0 = (id % p.row_blocks) * kG2Rows;
+    const int T0 = (id / p.row_blocks) * TT;
     const int nsb = p.K / kQK;
     const uint32_t xs0 = (uint32_t)(uintptr_t)&xs[0][0], wb0 = (uint32_t)(uintptr_t)&wb[0][0];
-    const uint32_t sb0 = (uint32_t)(uintptr_t)&sb_lds[0];
+    const uint32_t ss0 = (uint32_t)(uintptr_t)&ss[0][0];
 
     // ---- DMA plans (wave-uniform bases, per-lane offsets) ----
-    // activations: instruction i = kG2XInst * wave + r covers tokens 2i, 2i+1: lane ->
-    // token 2i + (lane >> 5), hi/lo (lane >> 4) & 1, LDS chunk lane & 15
+    // a token tile past the last one reads it and is never stored
+    auto tile = [&](int tt) { return T0 + tt < p.tiles ? T0 + tt : p.tiles - 1; };
+    // operand i = kG2XInst * wave + r of half h: sub-block, tile, hi or lo
     auto issue_x = [&](int h, int buf) {
 #pragma unroll
         for (int r = 0; r < kG2XInst; ++r) {
             const int i = kG2XInst * wave + r;
-            const int t = 2 * i + (lane >> 5);
-            const uint32_t off = (uint32_t)((lane >> 4) & 1) * p.xl_off +
-                                 (uint32_t)((t0 + t) * p.K + 128 * h) * 2u + 16u * (uint32_t)((lane & 15) ^ (t & 15));
-            dma16(off, p.x, xs0 + (uint32_t)(buf * kG2Half + 1024 * i));
+            dma16(16u * lane, p.xb + ((int64_t)tile((i >> 1) % TT) * (8 * nsb) + 4 * h + (i >> 1) / TT) * 128 + 64 * (i & 1),
+                  xs0 + (uint32_t)(buf * kG2Half + 1024 * i));
         }
     };
     // weights: chunk id = 64 * i + lane -> row id / 9, chunk id % 9 (rows past N
-    // read row 0 and are never stored)
-    uint32_t woff[kG2WPer];
+    // read the last one and are never stored)
+    uint32_t wrow[kG2WPer], wch[kG2WPer];
 #pragma unroll
     for (int r = 0; r < kG2WPer; ++r) {
         const int i = kG2Waves * r + wave;
-        const int id = 64 * (i < kG2WInst ? i : 0) + lane;
-        const int row = id / 9, ch = id - 9 * (id / 9);
-        const int grow = row0 + row < p.N ? row0 + row : 0;
-        woff[r] = (uint32_t)((int64_t)grow * p.w_nb1) + 16u * (uint32_t)ch;
+        const int c = 64 * (i < kG2WInst ? i : 0) + lane, row = row0 + c / 9;
+        wrow[r] = (uint32_t)((int64_t)((row < p.N ? row : p.N - 1) - row0) * p.w_nb1);
+        wch[r] = 16u * (uint32_t)(c % 9);
     }
+    const uint8_t *w0 = p.w + (int64_t)row0 * p.w_nb1;
     auto issue_w = [&](int sb, int buf) {
 #pragma unroll
         for (int r = 0; r < kG2WPer; ++r) {
             const int i = kG2Waves * r + wave;
-            if (i < kG2WInst) dma16(woff[r], p.w + (int64_t)sb * kBlockBytes, wb0 + (uint32_t)(buf * kG2WBytes + 1024 * i));
+            if (i < kG2WInst)
+                dma16(wrow[r] + wch[r], w0 + (int64_t)sb * kBlockBytes, wb0 + (uint32_t)(buf * kG2WBytes + 1024 * i));
         }
-    };
-    // S slots of group q into buffer q & 1: wavefront w < 4 copies tokens
-    // 8w..8w+7 (128 bytes each)
-    auto issue_s = [&](int q) {
-        if (wave >= kG2Tok / 8) return;
-        const int t = 8 * wave + (lane >> 3);
-        const uint32_t off = (uint32_t)(((t0 + t) * p.nq + q) * 128 + 16 * (lane & 7));
-        dma16(off, p.sp, sb0 + (uint32_t)((q & 1) * kG2SBytes + 1024 * wave));
+        if (wave < TT)
+            dma16(16u * lane, p.sb + ((int64_t)tile(wave) * nsb + sb) * 64, ss0 + (uint32_t)(buf * kG2SBytes + 1024 * wave));
     };
 
-    floatx4 acc[kG2RT][2], accm[kG2RT][2];
+    floatx4 acc[TT];
 #pragma unroll
-    for (int rt = 0; rt < kG2RT; ++rt)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) acc[rt][tt] = accm[rt][tt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    uint32_t amh[kG2RT][4], aml[kG2RT][4];  // A of the min MFMA per row tile: slots 2u, 2u+1 in dword u
-#pragma unroll
-    for (int rt = 0; rt < kG2RT; ++rt)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) amh[rt][u] = aml[rt][u] = 0u;
-
-    // Issue order: weights of super-blocks 0..kG2WAhead-1, S of group 0 and
-    // activation halves 0..kG2XAhead-1 first; then at the start of half k the
-    // weights of super-block k/2 + kG2WAhead (even k), the S of group k/8 + 1 (k a
-    // multiple of 8) and activation half k + kG2XAhead. A stage is read only after
-    // the wait for activation half h, and every DMA it needs was issued no later
-    // than that half's.
-    const int nh = 2 * nsb, ngrp = (nsb + 3) / 4;
-    for (int sb = 0; sb < kG2WAhead && sb < nsb; ++sb) issue_w(sb, sb);
-    issue_s(0);
-    for (int k = 0; k < kG2XAhead && k < nh; ++k) issue_x(k, k);
+    for (int tt = 0; tt < TT; ++tt) acc[tt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    issue_w(0, 0);
+    issue_x(0, 0);
     for (int sb = 0; sb < nsb; ++sb) {
-        const int u = sb & 3;
-        const uint8_t *wcur = &wb[sb % kG2WBufs][0];
-        int sc[kG2RT][8];
-        floatx4 dq[kG2RT];  // d 2^24 of C rows 4g..4g+3
-        floatx4 C[kG2RT][2];
+        const uint8_t *hrow = &wb[sb & 1][0] + (16 * wave + n) * kBlockBytes;
+        OpHead hd;
+        floatx4 C[TT];
 #pragma unroll
-        for (int rt = 0; rt < kG2RT; ++rt)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) C[rt][tt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int tt = 0; tt < TT; ++tt) C[tt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
             const int h = 2 * sb + hh;
-            // this wavefront's DMAs for half h have landed; the barrier publishes
-            // every wavefront's and retires the buffers the next DMAs overwrite.
-            // Half h's activations were the last DMA issued (at the start of half
-            // h - 1, after that half's weights and S slots), so the wait drains all.
+            // this wavefront's DMAs have landed (those of half h were the last it
+            // issued); the barrier publishes every wavefront's and retires the buffers
+            // that the next DMAs overwrite
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (hh == 0 && sb + kG2WAhead < nsb) issue_w(sb + kG2WAhead, (sb + kG2WAhead) % kG2WBufs);
-            if (hh == 0 && u == 0 && (sb >> 2) + 1 < ngrp) issue_s((sb >> 2) + 1);
-            if (h + kG2XAhead < nh) issue_x(h + kG2XAhead, (h + kG2XAhead) % kG2XBufs);
-            if (hh == 0) {
-                // scales of A row n (every sub-block), d of C rows 4g..4g+3, and
-                // this lane's two min slots (sub-blocks 2g, 2g+1)
-#pragma unroll
-                for (int rt = 0; rt < kG2RT; ++rt) {
-                    const uint8_t *hrow = wcur + (16 * kG2RT * wave + 16 * rt + n) * kBlockBytes;
-                    const uint4 hd = *reinterpret_cast<const uint4 *>(hrow);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        int mn;
-                        scale_min(hd.y, hd.z, hd.w, e, sc[rt][e], mn);
-                    }
-                    int m0, m1, unused;
-                    scale_min(hd.y, hd.z, hd.w, 2 * g, unused, m0);
-                    scale_min(hd.y, hd.z, hd.w, 2 * g + 1, unused, m1);
-                    const float dmin = h2f(hd.x >> 16);
-                    float a0 = dmin * (float)m0, a1 = dmin * (float)m1;  // exact: 11 x 6 bits
-                    asm volatile("" : "+v"(a0), "+v"(a1));
-                    const _Float16 h0 = (_Float16)a0, h1 = (_Float16)a1;
-                    const _Float16 l0 = (_Float16)(a0 - (float)h0), l1 = (_Float16)(a1 - (float)h1);
-                    uint16_t b[4];
-                    __builtin_memcpy(&b[0], &h0, 2);
-                    __builtin_memcpy(&b[1], &h1, 2);
-                    __builtin_memcpy(&b[2], &l0, 2);
-                    __builtin_memcpy(&b[3], &l1, 2);
-                    const uint32_t hw = (uint32_t)b[0] | ((uint32_t)b[1] << 16);
-                    const uint32_t lw = (uint32_t)b[2] | ((uint32_t)b[3] << 16);
-#pragma unroll
-                    for (int uu = 0; uu < 4; ++uu) {
-                        amh[rt][uu] = u == uu ? hw : amh[rt][uu];
-                        aml[rt][uu] = u == uu ? lw : aml[rt][uu];
-                    }
-                    float dv[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        dv[i] = h2f(*reinterpret_cast<const uint16_t *>(wcur + (16 * kG2RT * wave + 16 * rt + 4 * g + i) * kBlockBytes));
-                    dq[rt] = floatx4{dv[0], dv[1], dv[2], dv[3]} * 16777216.0f;
-                }
-            }
-            const uint8_t *xb = &xs[h % kG2XBufs][0];
+            if (hh == 0 && sb + 1 < nsb) issue_w(sb + 1, (sb + 1) & 1);
+            if (h + 1 < 2 * nsb) issue_x(h + 1, (h + 1) & 1);
+            if (hh == 0) hd = op_head(*reinterpret_cast<const uint4 *>(hrow), g);
+            const uint4 w = *reinterpret_cast<const uint4 *>(hrow + 16 + 32 * g + 16 * hh);
+            const uint8_t *xb = &xs[h & 1][0] + 16 * lane;
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj) {
-                const int j = 2 * hh + jj;  // code group: sub-blocks 2j (low nibbles), 2j+1 (high)
-                half8 alo[kG2RT], ahi[kG2RT];
+                half8 a[2], b[TT][4];  // step 2 hh + jj
+                op_a_operand(hd, jj ? w.z : w.x, jj ? w.w : w.y, a[0], a[1]);
 #pragma unroll
-                for (int rt = 0; rt < kG2RT; ++rt) {
-                    const uint2 qv = *reinterpret_cast<const uint2 *>(wcur + (16 * kG2RT * wave + 16 * rt + n) * kBlockBytes +
-                                                                      16 + 32 * j + 8 * g);
-                    uint32_t sp4[4];  // bytes 2m, 2m+1 spread to the two halves of dword m
-                    sp4[0] = __builtin_amdgcn_perm(0u, qv.x, 0x0c010c00u);
-                    sp4[1] = __builtin_amdgcn_perm(0u, qv.x, 0x0c030c02u);
-                    sp4[2] = __builtin_amdgcn_perm(0u, qv.y, 0x0c010c00u);
-                    sp4[3] = __builtin_amdgcn_perm(0u, qv.y, 0x0c030c02u);
-                    uint32_t lo[4], hi[4];
+                for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) {
-                        lo[m] = __umul24(sp4[m] & 0x000F000Fu, (uint32_t)sc[rt][2 * j]);
-                        hi[m] = __umul24((sp4[m] >> 4) & 0x000F000Fu, (uint32_t)sc[rt][2 * j + 1]);
-                    }
-                    __builtin_memcpy(&alo[rt], lo, 16);
-                    __builtin_memcpy(&ahi[rt], hi, 16);
-                }
+                    for (int c = 0; c < 4; ++c)
+                        b[tt][c] = *reinterpret_cast<const half8 *>(
+                            xb + (((2 * jj + (c >> 1)) * TT + tt) * 2 + (c & 1)) * 1024);
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const int tr = 16 * tt + n;
-                    const uint8_t *row = xb + 512 * tr;
-                    const int c0 = 8 * jj + g, c1 = 8 * jj + 4 + g;
-                    half8 bh0, bl0, bh1, bl1;
-                    {
-                        const uint4 a = *reinterpret_cast<const uint4 *>(row + 16 * (c0 ^ (tr & 15)));
-                        const uint4 b = *reinterpret_cast<const uint4 *>(row + 256 + 16 * (c0 ^ (tr & 15)));
-                        const uint4 c = *reinterpret_cast<const uint4 *>(row + 16 * (c1 ^ (tr & 15)));
-                        const uint4 d = *reinterpret_cast<const uint4 *>(row + 256 + 16 * (c1 ^ (tr & 15)));
-                        __builtin_memcpy(&bh0, &a, 16);
-                        __builtin_memcpy(&bl0, &b, 16);
-                        __builtin_memcpy(&bh1, &c, 16);
-                        __builtin_memcpy(&bl1, &d, 16);
-                    }
+                for (int c = 0; c < 4; ++c)
 #pragma unroll
-                    for (int rt = 0; rt < kG2RT; ++rt) {
-                        C[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[rt], bh0, C[rt][tt], 0, 0, 0);
-                        C[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[rt], bl0, C[rt][tt], 0, 0, 0);
-                        C[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[rt], bh1, C[rt][tt], 0, 0, 0);
-                        C[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[rt], bl1, C[rt][tt], 0, 0, 0);
-                    }
-                }
+                    for (int tt = 0; tt < TT; ++tt)
+                        C[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c >> 1], b[tt][c], C[tt], 0, 0, 0);
             }
         }
+        uint4 sv[TT];
 #pragma unroll
-        for (int rt = 0; rt < kG2RT; ++rt)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[rt][tt][i] = fmaf(dq[rt][i], C[rt][tt][i], acc[rt][tt][i]);
-        // min MFMA at the end of a group of four super-blocks (or of K)
-        if (u == 3 || sb == nsb - 1) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const uint8_t *srow = sb_lds + ((sb >> 2) & 1) * kG2SBytes + 128 * (16 * tt + n);
-                const uint4 bhv = *reinterpret_cast<const uint4 *>(srow + 16 * g);
-                const uint4 blv = *reinterpret_cast<const uint4 *>(srow + 64 + 16 * g);
-                half8 bh, bl;
-                __builtin_memcpy(&bh, &bhv, 16);
-                __builtin_memcpy(&bl, &blv, 16);
-#pragma unroll
-                for (int rt = 0; rt < kG2RT; ++rt) {
-                    half8 ah, al;
-                    __builtin_memcpy(&ah, amh[rt], 16);
-                    __builtin_memcpy(&al, aml[rt], 16);
-                    accm[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, accm[rt][tt], 0, 0, 0);
-                    accm[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, accm[rt][tt], 0, 0, 0);
-                    accm[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, accm[rt][tt], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int rt = 0; rt < kG2RT; ++rt)
-#pragma unroll
-                for (int uu = 0; uu < 4; ++uu) amh[rt][uu] = aml[rt][uu] = 0u;
-        }
+        for (int tt = 0; tt < TT; ++tt)
+            sv[tt] = *reinterpret_cast<const uint4 *>(&ss[sb & 1][0] + 1024 * tt + 16 * lane);
+        op_scale_add<TT>(hd, g, C, sv, acc);
     }
-    // ---- out[token][rows 4g..4g+3] = acc - accm ----
+    const int r = row0 + 16 * wave;
+    if (r >= p.N) return;
 #pragma unroll
-    for (int rt = 0; rt < kG2RT; ++rt) {
-        const int r = row0 + 16 * kG2RT * wave + 16 * rt;
-        if (r >= p.N) continue;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int t = t0 + 16 * tt + n;
-            if (t >= p.M) continue;
-            float *drow = reinterpret_cast<float *>(reinterpret_cast<char *>(p.dst) + (int64_t)t * p.d_nb1);
-            const floatx4 o = acc[rt][tt] - accm[rt][tt];
-            *reinterpret_cast<float4 *>(drow + r + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
-        }
+    for (int tt = 0; tt < TT; ++tt) {
+        const int t = 16 * (T0 + tt) + n;
+        if (t < p.M)
+            *reinterpret_cast<float4 *>(reinterpret_cast<char *>(p.dst) + (int64_t)t * p.d_nb1 + 4 * (r + 4 * g)) =
+                make_float4(acc[tt][0], acc[tt][1], acc[tt][2], acc[tt][3]);
     }
 }
 
@@ -811,22 +697,17 @@ __global__ __launch_bounds__(kGemvThreads) void op_gemv_kernel(const uint8_t *__
     }
 }
 
-size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-// Workspace of the GEMM path: tokens padded to Mp (a multiple of 32), xh and xl
-// [Mp][K] fp16, S [Mp][K/32] f32, the S hi/lo slots [Mp][nq][64] fp16.
+// Workspace of the GEMM path (see op_prep): 2 KB of x operands per 16 tokens and
+// sub-block, 1 KB of S operands per 16 tokens and super-block.
 struct OpLayout {
-    int64_t Mp, nq;
-    size_t xl, s, sp, total;
+    int64_t tiles;
+    size_t sb, total;
 };
 OpLayout op_layout(int64_t K, int64_t M) {
     OpLayout l;
-    l.Mp = (M + kG2Tok - 1) / kG2Tok * kG2Tok;
-    l.nq = (K / kQK + 3) / 4;
-    l.xl = al256((size_t)(l.Mp * K) * 2);
-    l.s = 2 * l.xl;
-    l.sp = l.s + al256((size_t)(l.Mp * (K / 32)) * 4);
-    l.total = l.sp + al256((size_t)(l.Mp * l.nq * 64) * 2) + 256;
+    l.tiles = (M + 15) / 16;
+    l.sb = (size_t)(l.tiles * (K / 32)) * 2048;
+    l.total = l.sb + (size_t)(l.tiles * (K / kQK)) * 1024 + 256;
     return l;
 }
 
@@ -869,76 +750,68 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     if (!ws || ws_bytes < need)
         return set_error(SQA_ERR_WORKSPACE, "out_proj: workspace %zu bytes < %zu needed", ws_bytes, need);
     uint8_t *base = reinterpret_cast<uint8_t *>(((uintptr_t)ws + 255) & ~(uintptr_t)255);
-    uint16_t *xh = reinterpret_cast<uint16_t *>(base);
-    uint16_t *xl = reinterpret_cast<uint16_t *>(base + L.xl);
-    float *S = reinterpret_cast<float *>(base + L.s);
-    uint16_t *sp = reinterpret_cast<uint16_t *>(base + L.sp);
-    // op_gemm2 once there are enough 32-token tiles to fill the chip; its DMA
-    // offsets are 32-bit
-    const bool big = M > 64 && (uint64_t)L.xl * 2 < (1ull << 32) && (uint64_t)N * w.nb[1] < (1ull << 32);
-    if (big) {
-        static std::once_flag g2_once;
-        static hipError_t g2_err = hipSuccess;
-        std::call_once(g2_once, [] {
-            g2_err = hipFuncSetAttribute((const void *)op_gemm2_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kG2Lds);
-        });
-        if (g2_err != hipSuccess) return hip_status(g2_err, "out_proj LDS attribute");
-    }
+    uint4 *xb = reinterpret_cast<uint4 *>(base), *sb = reinterpret_cast<uint4 *>(base + L.sb);
+    static std::once_flag g2_once;
+    static hipError_t g2_err = hipSuccess;
+    std::call_once(g2_once, [] {
+        g2_err = hipFuncSetAttribute((const void *)op_gemm2_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kG2Lds);
+    });
+    if (g2_err != hipSuccess) return hip_status(g2_err, "out_proj LDS attribute");
 
     const int prof = profile_start("out_proj", s);
-    const int64_t nprep = 4 * 32 * L.nq * L.Mp;
     const bool vec = (uintptr_t)x.data % 16 == 0 && x.nb[1] % 16 == 0 &&
                      (!gate || ((uintptr_t)gate->data % 16 == 0 && gate->nb[1] % 16 == 0));
-    const dim3 pg((unsigned)((nprep + 255) / 256));
+    const dim3 pg((unsigned)((L.tiles * (K / 64) + 3) / 4));
     const char *xd = (const char *)x.data, *gd = gate ? (const char *)gate->data : nullptr;
     const int64_t xn = (int64_t)x.nb[1], gn = gate ? (int64_t)gate->nb[1] : 0;
-    const int Ki = (int)K, Mi = (int)M, Mpi = (int)L.Mp, nqi = (int)L.nq;
+    const int Ki = (int)K, Mi = (int)M, tl = (int)L.tiles;
     if (gate && vec)
-        op_prep_kernel<true, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, Mpi, nqi, xh, xl, S, sp);
+        op_prep_kernel<true, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
     else if (gate)
-        op_prep_kernel<true, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, Mpi, nqi, xh, xl, S, sp);
+        op_prep_kernel<true, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
     else if (vec)
-        op_prep_kernel<false, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, Mpi, nqi, xh, xl, S, sp);
+        op_prep_kernel<false, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
     else
-        op_prep_kernel<false, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, Mpi, nqi, xh, xl, S, sp);
-    if (big) {
-        Gemm2Params q;
-        q.w = (const uint8_t *)w.data;
-        q.w_nb1 = (int64_t)w.nb[1];
-        q.x = xh;
-        q.xl_off = (uint32_t)L.xl;
-        q.sp = sp;
-        q.K = Ki;
-        q.N = (int)N;
-        q.M = Mi;
-        q.Mp = Mpi;
-        q.nq = nqi;
-        q.dst = (float *)dst.data;
-        q.d_nb1 = (int64_t)dst.nb[1];
-        op_gemm2_kernel<<<dim3((unsigned)((N + kG2Rows - 1) / kG2Rows), (unsigned)(L.Mp / kG2Tok)), dim3(64 * kG2Waves), kG2Lds,
-                          s>>>(q);
+        op_prep_kernel<false, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
+    GemmParams p;
+    p.w = (const uint8_t *)w.data;
+    p.w_nb1 = (int64_t)w.nb[1];
+    p.xb = xb;
+    p.sb = sb;
+    p.K = Ki;
+    p.N = (int)N;
+    p.M = Mi;
+    p.tiles = tl;
+    p.dst = (float *)dst.data;
+    p.d_nb1 = (int64_t)dst.nb[1];
+#define SQA_GEMM(KS, RT, TT)                                                                                \
+    do {                                                                                                    \
+        p.row_blocks = (int)((N + 16 * RT - 1) / (16 * RT));                                                \
+        op_gemm_kernel<KS, RT, TT><<<dim3((unsigned)(p.row_blocks * ((tl + TT - 1) / TT))), dim3(64 * KS), 0, \
+                                     s>>>(p);                                                              \
+    } while (0)
+    // units of 16 rows x 16 tokens. Few of them: the smallest workgroup tile of
+    // op_gemm that still leaves at most one workgroup per CU (with two the time
+    // doubles); more: op_gemm2. us at N = 2048, K = 4096 with op_prep, op_gemm
+    // <16, 1, 1> / <16, 1, 2> / <16, 2, 2> / <8, 4, 2> / op_gemm2: 23 tokens 9.9 / 12.3 /
+    // 14.3 / 20.5 / 28.1, 64 tokens 13.8 / 13.0 / 14.4 / 20.5 / 28.2, 128 tokens 23.1 /
+    // 20.4 / 15.4 / 20.9 / 28.6, 256 tokens 39 / 36 / 27.6 / 23.6 / 30.6, 300 tokens 46 /
+    // 43 / 36 / 38 / 31.9, 512 tokens 70 / 62 / 46 / 41 / 32.8. op_gemm2's DMA
+    // addresses its 128 rows with 32-bit offsets.
+    const int64_t cus = device_cu_count(), units = N / 16 * L.tiles;
+    if (units <= cus) {
+        SQA_GEMM(16, 1, 1);
+    } else if (units <= 2 * cus) {
+        SQA_GEMM(16, 1, 2);
+    } else if (units <= 4 * cus) {
+        SQA_GEMM(16, 2, 2);
+    } else if (units <= 8 * cus || (uint64_t)kG2Rows * w.nb[1] >= (1ull << 32)) {
+        SQA_GEMM(8, 4, 2);
     } else {
-        const int64_t M16 = (M + 15) / 16 * 16;
-        GemmParams p;
-        p.w = (const uint8_t *)w.data;
-        p.w_nb1 = (int64_t)w.nb[1];
-        p.xh = xh;
-        p.xl = xl;
-        p.S = S;
-        p.K = Ki;
-        p.N = (int)N;
-        p.M = Mi;
-        p.M16 = (int)M16;
-        p.dst = (float *)dst.data;
-        p.d_nb1 = (int64_t)dst.nb[1];
-        // one 16-token tile per workgroup; for decode (one token tile) 16 rows and
-        // 16 wavefronts that take one super-block each, else 64 rows and 4 wavefronts
-        if (M16 == 16 || N % 64 != 0)
-            op_gemm_kernel<16, 1><<<dim3((unsigned)(N / 16), (unsigned)(M16 / 16)), dim3(1024), 0, s>>>(p);
-        else
-            op_gemm_kernel<4, 4><<<dim3((unsigned)(N / 64), (unsigned)(M16 / 16)), dim3(256), 0, s>>>(p);
+        p.row_blocks = (int)((N + kG2Rows - 1) / kG2Rows);
+        op_gemm2_kernel<<<dim3((unsigned)(p.row_blocks * ((tl + kG2TT - 1) / kG2TT))), dim3(64 * kG2Waves), kG2Lds, s>>>(p);
     }
+#undef SQA_GEMM
     profile_stop(prof, s);
     return hip_status(hipGetLastError(), "out_proj launch");
 }

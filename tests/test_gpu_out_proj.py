@@ -109,3 +109,12 @@ def test_out_proj_rejects_unsupported_shapes(sqa, dev):
     x = torch.zeros((1, 256), device=dev)
     with pytest.raises(sqa.SqaError):
         sqa.out_proj(w, x)
+
+
+@pytest.mark.parametrize("K", [256, 1792])
+@pytest.mark.parametrize("M", [5, 32, 33, 64, 65, 128, 129, 256, 257])
+def test_out_proj_tile_rule_edges(sqa, orc, dev, M, K):
+    # both sides of every step of the tile rule at 128 row tiles (256 to 2048 units
+    # of 16 rows x 16 tokens on 256 CUs), last token tiles full and ragged, one
+    # super-block and 7 (fewer than and not a multiple of the K splits)
+    assert run(sqa, orc, dev, 2048, K, M, 300 + M + K, outliers=4) <= TOL
