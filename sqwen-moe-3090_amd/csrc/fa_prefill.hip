@@ -132,9 +132,8 @@ __device__ __forceinline__ int key_row(int k) { return 16 * ((k >> 2) & 1) + 4 *
 //      its 32 codes as fp16 (4 swizzled 16-byte chunks of the key's row) and its
 //      scale into the Dk row of block b;
 //   V: thread t writes the Vc row of dim t (32 codes, 64 bytes) of both tiles;
-//      threads 0..15 write the Dv rows and fold the largest |d_v| into
-//      dvmax[head] (fp16 magnitude bits, cleared by qprep_kernel, which runs
-//      first).
+//      the first wavefront writes the Dv rows and the group's largest |d_v|
+//      (fp16 magnitude bits) into dvmax[head][group].
 // N dwords of a q4_0 block's qs bytes starting at byte off (2 mod 4 for even
 // blocks, 0 mod 4 for odd ones) of an LDS row: aligned reads, shifted by
 // alignbit. Every read stays inside the row's 144 bytes.
@@ -164,14 +163,23 @@ __device__ __forceinline__ uint32_t codes_f16(uint32_t x) {
     return r;
 }
 
-__global__ __launch_bounds__(256) void kvprep_kernel(const uint8_t *__restrict__ k, int64_t k_nb1, int64_t k_nb2,
-                                                     const uint8_t *__restrict__ v, int64_t v_nb1, int64_t v_nb2,
-                                                     int64_t n_kv, int64_t kv_tiles, uint8_t *__restrict__ kv,
-                                                     uint32_t *__restrict__ dvmax) {
+struct KvPrep {
+    const uint8_t *k, *v;
+    int64_t k_nb1, k_nb2, v_nb1, v_nb2;
+    int64_t n_kv, kv_tiles;
+    int hkv, groups;   // KV heads; 64-key groups per head
+    uint8_t *kv;
+    uint32_t *dvmax;   // [hkv][groups]
+};
+
+__device__ __forceinline__ void kvprep(const KvPrep &p, int group, int h) {
     __shared__ __align__(16) uint8_t sk[64 * kHeadRowBytes], sv[64 * kHeadRowBytes];
     const int t = threadIdx.x;
-    const int h = blockIdx.y;
-    const int64_t k0 = (int64_t)blockIdx.x * 64;
+    const int64_t k0 = (int64_t)group * 64;
+    const uint8_t *k = p.k, *v = p.v;
+    uint8_t *kv = p.kv;
+    const int64_t k_nb1 = p.k_nb1, k_nb2 = p.k_nb2, v_nb1 = p.v_nb1, v_nb2 = p.v_nb2, n_kv = p.n_kv,
+                  kv_tiles = p.kv_tiles;
     for (int idx = t; idx < 64 * 9; idx += 256) {  // 9 x 16 bytes per 144-byte row
         const int key = idx / 9, c = idx - 9 * key;
         uint4 a = make_uint4(0, 0, 0, 0), b = make_uint4(0, 0, 0, 0);
@@ -273,7 +281,7 @@ __global__ __launch_bounds__(256) void kvprep_kernel(const uint8_t *__restrict__
                 const uint32_t other = (uint32_t)__shfl_xor((int)dmax, o);
                 dmax = other > dmax ? other : dmax;
             }
-            if (t == 0) atomicMax(dvmax + h, dmax);
+            if (t == 0) p.dvmax[(int64_t)h * p.groups + group] = dmax;
         }
     }
 }
@@ -344,26 +352,32 @@ __global__ __launch_bounds__(256) void mask_tile_limit_kernel(const char *__rest
     mask_tile_limit(mask, nb1, len, n_q, qb, blockIdx.x, lim);
 }
 
-// Workgroups from n_qblocks on are the mask scan (mask_tile_limit) of query
-// tile blockIdx.x - n_qblocks, when the kernel reads the caller's mask in place.
+// The mask scan (mask_tile_limit) of every query tile, when the kernel reads the
+// caller's mask in place.
 struct MaskScan {
     const char *mask;  // null: no scan here
     int64_t nb1, len;
-    int qb, n_qblocks;
+    int qb, tiles;
     int32_t *lim;
 };
 
-__global__ __launch_bounds__(256) void qprep_kernel(const char *__restrict__ q, int64_t nb1, int64_t nb2,
-                                                    int n_q, int H, float qscale, uint16_t *__restrict__ qh,
-                                                    uint16_t *__restrict__ ql, uint32_t *__restrict__ dvmax, int hkv,
-                                                    bool aligned, MaskScan ms) {
-    if (ms.mask && (int)blockIdx.x >= ms.n_qblocks) {
-        mask_tile_limit(ms.mask, ms.nb1, ms.len, n_q, ms.qb, (int)blockIdx.x - ms.n_qblocks, ms.lim);
-        return;
-    }
+struct QPrep {
+    const char *q;
+    int64_t nb1, nb2;
+    int n_q, H;
+    float qscale;
+    uint16_t *qh, *ql;
+    bool aligned;
+};
+
+__device__ __forceinline__ void qprep(const QPrep &p, int64_t gid) {
+    const char *q = p.q;
+    const int64_t nb1 = p.nb1, nb2 = p.nb2;
+    const int n_q = p.n_q, H = p.H;
+    const float qscale = p.qscale;
+    uint16_t *qh = p.qh, *ql = p.ql;
+    const bool aligned = p.aligned;
     // one thread per 8 values: a quad of lanes owns a 32-value block
-    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gid < hkv) dvmax[gid] = 0;  // for kvprep_kernel, launched next
     if (gid >= (int64_t)n_q * H * kBlocksPerHead * 4) return;  // whole quads: the total is a multiple of 4
     const int qtr = (int)(gid & 3);
     const int64_t bid = gid >> 2;
@@ -412,6 +426,28 @@ __global__ __launch_bounds__(256) void qprep_kernel(const char *__restrict__ q, 
     *reinterpret_cast<uint4 *>(ql + row * kHeadDim + 32 * b + 8 * qtr) = c;
 }
 
+// The pre-passes in one launch: the K/V groups first (the longest workgroups),
+// then the mask scans, then Q. As two launches, with the scans beside Q, they took
+// 8.3 + 5.1 us for 512 queries on 512 keys (8.4 now), 6.5 + 17 on 16896 keys
+// (16.8), 4.7 + 17.7 for 37 on 20048 (17.1), and the gap between them.
+__global__ __launch_bounds__(256) void prep_kernel(KvPrep kv, QPrep q, MaskScan ms) {
+    int id = (int)blockIdx.x;
+    const int n_kv = kv.groups * kv.hkv;
+    if (id < n_kv) {
+        kvprep(kv, id % kv.groups, id / kv.groups);
+        return;
+    }
+    id -= n_kv;
+    if (ms.mask) {
+        if (id < ms.tiles) {
+            mask_tile_limit(ms.mask, ms.nb1, ms.len, q.n_q, ms.qb, id, ms.lim);
+            return;
+        }
+        id -= ms.tiles;
+    }
+    qprep(q, (int64_t)id * 256 + threadIdx.x);
+}
+
 // Copies an F16 mask whose rows are unaligned or whose length is not a
 // multiple of 8 into [n_q][len8] rows (len8 = n_kv rounded up to 8, -inf pad).
 __global__ __launch_bounds__(256) void pf_mask_pack_kernel(const char *__restrict__ src, int64_t nb1, int64_t n_kv,
@@ -449,7 +485,7 @@ __device__ __forceinline__ half8 lds_half8(const uint8_t *base, int off_lo, int 
 
 struct PrefillParams {
     const uint8_t *kv;        // [Hkv][kv_tiles] tile records
-    const uint32_t *dvmax;    // [Hkv] fp16 magnitude bits
+    const uint32_t *dvmax;    // [Hkv][kv_tiles / 2] fp16 magnitude bits
     const uint16_t *qh, *ql;  // [n_q*H][256] fp16 Q' hi and lo
     int64_t n_kv, kv_tiles;
     int n_q, H, G, Hkv;
@@ -571,10 +607,25 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
     };
     if (n_tiles > 0) issue(0, -1);
 
+    // the head's largest |d_v| over its 64-key groups, by every wavefront for itself
+    uint32_t dv = 0;
+    {
+        const int groups = (int)(p.kv_tiles >> 1);
+        const uint32_t *m = p.dvmax + (int64_t)kvh * groups;
+        for (int i = lane; i < groups; i += 256) {
+            uint32_t a[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = i + 64 * j < groups ? m[i + 64 * j] : 0u;
+            dv = max(max(dv, max(a[0], a[1])), max(a[2], a[3]));
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) dv = max(dv, (uint32_t)__shfl_xor((int)dv, o));
+        dv = (uint32_t)__builtin_amdgcn_readfirstlane((int)dv);
+    }
     // e2 with max |d_v| * 2^e2 in [1, 2) (at most 15)
     int e2 = 0;
     {
-        const float dm = h2f(p.dvmax[kvh]);
+        const float dm = h2f(dv);
         if (dm > 0.0f) {
             int e;
             (void)frexpf(dm, &e);
@@ -1061,7 +1112,7 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     const int G = (int)(H / Hkv);
     pl.qb = kRowsPerWG / G;
     pl.mask_stage = pl.qb * kPK * 2;
-    pl.kv_tiles = (n_kv + 63) / 64 * 2;  // vdeq writes 64-key groups
+    pl.kv_tiles = (n_kv + 63) / 64 * 2;  // the pre-pass writes 64-key groups
     pl.q_tiles = (int)((n_q + pl.qb - 1) / pl.qb);
     pl.split_len = split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H);
     pl.n_splits = (int)((n_kv + pl.split_len - 1) / pl.split_len);
@@ -1070,7 +1121,7 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     const int64_t parts = max_splits(n_kv, pl.q_tiles * Hkv);
     size_t o = 0;
     pl.off_kv = o; o = al256(o + (size_t)Hkv * pl.kv_tiles * kTileBytes);
-    pl.off_dvmax = o; o = al256(o + (size_t)Hkv * 4);
+    pl.off_dvmax = o; o = al256(o + (size_t)Hkv * (size_t)(pl.kv_tiles / 2) * 4);
     pl.off_qh = o; o = al256(o + (size_t)n_q * H * kHeadDim * 2);
     pl.off_ql = o; o = al256(o + (size_t)n_q * H * kHeadDim * 2);
     pl.off_mask = o; o = al256(o + (size_t)n_q * ((n_kv + 7) / 8 * 8) * 2);
@@ -1138,15 +1189,16 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
         const int64_t nqb = n_q * H * kBlocksPerHead;
         const int qblocks = (int)((4 * nqb + 255) / 256);
         int32_t *lim = reinterpret_cast<int32_t *>(base + pl.off_lim);
-        // an in-place mask is scanned by extra workgroups of the Q pre-pass, a
-        // packed copy by a kernel of its own once it is written
-        const MaskScan ms{p.mask && !mask_src ? p.mask : nullptr, p.mask_nb1, p.mask_len, pl.qb, qblocks, lim};
-        qprep_kernel<<<dim3((unsigned)(qblocks + (ms.mask ? pl.q_tiles : 0))), dim3(256), 0, s>>>(
-            (const char *)q.data, (int64_t)q.nb[1], (int64_t)q.nb[2], (int)n_q, (int)H, a.scale * kLog2e, qh, ql,
-            dvmax, (int)Hkv, (uintptr_t)q.data % 16 == 0 && q.nb[1] % 16 == 0 && q.nb[2] % 16 == 0, ms);
-        kvprep_kernel<<<dim3((unsigned)(pl.kv_tiles / 2), (unsigned)Hkv), dim3(256), 0, s>>>(
-            (const uint8_t *)k.data, (int64_t)k.nb[1], (int64_t)k.nb[2], (const uint8_t *)v.data, (int64_t)v.nb[1],
-            (int64_t)v.nb[2], n_kv, pl.kv_tiles, kv, dvmax);
+        // an in-place mask is scanned by extra workgroups of the pre-pass, a packed
+        // copy by a kernel of its own once it is written
+        const MaskScan ms{p.mask && !mask_src ? p.mask : nullptr, p.mask_nb1, p.mask_len, pl.qb, pl.q_tiles, lim};
+        const QPrep qp{(const char *)q.data, (int64_t)q.nb[1], (int64_t)q.nb[2], (int)n_q, (int)H, a.scale * kLog2e,
+                       qh, ql, (uintptr_t)q.data % 16 == 0 && q.nb[1] % 16 == 0 && q.nb[2] % 16 == 0};
+        const KvPrep kp{(const uint8_t *)k.data, (const uint8_t *)v.data, (int64_t)k.nb[1], (int64_t)k.nb[2],
+                        (int64_t)v.nb[1], (int64_t)v.nb[2], n_kv, pl.kv_tiles, (int)Hkv, (int)(pl.kv_tiles / 2), kv,
+                        dvmax};
+        prep_kernel<<<dim3((unsigned)(kp.groups * kp.hkv + (ms.mask ? pl.q_tiles : 0) + qblocks)), dim3(256), 0, s>>>(
+            kp, qp, ms);
         if (mask_src) {
             int64_t grid = (p.mask_len * n_q + 255) / 256;
             if (grid > 2048) grid = 2048;
