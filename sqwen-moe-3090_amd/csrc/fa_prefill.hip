@@ -17,7 +17,7 @@
 // swizzled, see below), so its K and V halves move HBM -> LDS as straight
 // copies. Keys past n_kv are zero.
 //
-// fa_prefill_kernel: a workgroup takes 128 query rows of ONE KV head (GQA
+// fa_prefill_kernel: a workgroup takes 128 (or 64) query rows of ONE KV head (GQA
 // packed: row r is position r / G, head kvh*G + r % G) and streams 32-key
 // tiles. Its 8 wavefronts (2 per SIMD) split the work by kind:
 //   score wave w (0..3), rows 32w..32w+31, holds their Q' hi and lo (128
@@ -73,8 +73,8 @@ constexpr int kScoreWaves = 4;           // 32 rows each
 constexpr int kValueWaves = 4;           // 32 rows each
 constexpr int kWaves = kScoreWaves + kValueWaves;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kRG = 2;                   // 16-row groups per score wave
-constexpr int kRowsPerWG = kScoreWaves * kRG * 16;  // 128 query rows
+constexpr int kMaxRG = 2;                // 16-row groups per score wave: 1 or 2 (kRG in the kernel)
+constexpr int rows_per_wg(int rg) { return kScoreWaves * rg * 16; }  // 64 or 128 query rows
 constexpr int kOffDk = kPK * 512;        // inside the K half: Dk after Kc
 constexpr int kKHalf = kOffDk + 8 * kPK * 2;  // Kc + Dk: 16896 bytes
 constexpr int kOffDv = kHeadDim * kPK * 2;  // inside the V half: Dv after Vc
@@ -83,12 +83,12 @@ constexpr int kTileBytes = kKHalf + kVHalf;   // one tile record
 constexpr int kKInst = (kKHalf + 1023) / 1024;  // 17 DMA instructions, the last one 512 bytes
 constexpr int kVInst = (kVHalf + 1023) / 1024;  // 17, the last one 512 bytes
 constexpr int kKStage = kKInst * 1024, kVStage = kVInst * 1024;
-// LDS map: 2 K stages | 2 V stages | 2 P buffers | 2 rescale buffers | 2 mask stages
+// LDS map (sized for kMaxRG): 2 K stages | 2 V stages | 2 P buffers | 2 rescale buffers | 2 mask stages
 constexpr int kLdsV = 2 * kKStage;
 constexpr int kLdsP = kLdsV + 2 * kVStage;        // [4 waves][2 rg][2 halves][64 lanes][16 B]
-constexpr int kPBuf = kScoreWaves * kRG * 2 * 1024;
+constexpr int kPBuf = kScoreWaves * kMaxRG * 2 * 1024;
 constexpr int kLdsA = kLdsP + 2 * kPBuf;          // [4 waves][2 rg][16 rows] f32
-constexpr int kABuf = kScoreWaves * kRG * 16 * 4;
+constexpr int kABuf = kScoreWaves * kMaxRG * 16 * 4;
 constexpr int kLdsMask = kLdsA + 2 * kABuf;       // [qb positions][32 keys] f16
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kSlack = 8;  // log2 of the largest P the lazy rescale admits (V not large)
@@ -505,6 +505,8 @@ struct PrefillParams {
     int64_t gate_nb1, gate_nb2;
 };
 
+// kRG = 2: 128 query rows; 1: 64 rows (see plan for where).
+template <int kRG>
 __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x;
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         // a split past the tile's last visible key leaves its O unwritten: the
         // merge takes no partial whose m is -inf
         const int pos = q_base + tid / p.G;
-        if (tid < kRowsPerWG && pos < p.n_q) {
+        if (tid < rows_per_wg(kRG) && pos < p.n_q) {
             const int64_t row = (int64_t)split * p.n_q * p.H + (int64_t)pos * p.H + kvh * p.G + tid % p.G;
             store_through(p.part_ml + row * 2, -INFINITY);
             store_through(p.part_ml + row * 2 + 1, 0.0f);
@@ -669,7 +671,7 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         float mref[kRG], lim_s[kRG];
 #pragma unroll
         for (int rg = 0; rg < kRG; ++rg) {
-            const int r = 32 * w + 16 * rg + n;
+            const int r = 16 * kRG * w + 16 * rg + n;
             const int pos = q_base + r / p.G;
             my_pos[rg] = pos;
             const bool ok = pos < p.n_q;
@@ -977,7 +979,7 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
     for (int rg = 0; rg < kRG; ++rg) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = 32 * w + 16 * rg + 4 * g + i;
+            const int r = 16 * kRG * w + 16 * rg + 4 * g + i;
             const int qrow = q_base + r / p.G, hrow = kvh * p.G + r % p.G;
             if (qrow >= p.n_q) continue;
             const float mrow = n_tiles > 0 ? ml[rg * 32 + 2 * (4 * g + i)] : -INFINITY;
@@ -1015,7 +1017,7 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct PrefillPlan {
     int64_t kv_tiles;
-    int qb, q_tiles, n_splits, mask_stage;
+    int rg, qb, q_tiles, n_splits, mask_stage;
     int64_t split_len;
     size_t off_kv, off_dvmax, off_qh, off_ql, off_mask, off_lim, off_pa, off_pm, total;
 };
@@ -1110,7 +1112,15 @@ int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q
 PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     PrefillPlan pl{};
     const int G = (int)(H / Hkv);
-    pl.qb = kRowsPerWG / G;
+    // 64-row workgroups where 128 rows would leave most of their work to padding or
+    // most of the chip idle: a query tile of all the rows, and an unsplit chunk
+    // whose 64-row workgroups still run in one round. A tile of keys costs them
+    // about 1.5 us where 128 rows take 2.2 to 2.4: us per call 128 rows / 64 rows 512
+    // first queries 48.3 / 35.1, 200 first queries 32.3 / 21.5, 8 on 3008 keys 34 / 24.
+    const int64_t cus = device_cu_count();
+    const int64_t wgs64 = (n_q + rows_per_wg(1) / G - 1) / (rows_per_wg(1) / G) * Hkv;
+    pl.rg = n_q * G <= rows_per_wg(1) || (n_kv <= kOneSplitKeys && wgs64 <= cus) ? 1 : 2;
+    pl.qb = rows_per_wg(pl.rg) / G;
     pl.mask_stage = pl.qb * kPK * 2;
     pl.kv_tiles = (n_kv + 63) / 64 * 2;  // the pre-pass writes 64-key groups
     pl.q_tiles = (int)((n_q + pl.qb - 1) / pl.qb);
@@ -1244,12 +1254,19 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     static std::once_flag lds_once;
     static hipError_t lds_err = hipSuccess;
     std::call_once(lds_once, [] {
-        lds_err = hipFuncSetAttribute((const void *)fa_prefill_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        lds_err = hipFuncSetAttribute((const void *)fa_prefill_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       kLdsMaxBytes);
+        if (lds_err == hipSuccess)
+            lds_err = hipFuncSetAttribute((const void *)fa_prefill_kernel<2>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMaxBytes);
     });
     if (lds_err != hipSuccess) return hip_status(lds_err, "fa_prefill LDS attribute");
     prof = profile_start("fa_prefill", s);
-    fa_prefill_kernel<<<dim3((unsigned)(pl.q_tiles * Hkv * pl.n_splits)), dim3(kThreads), lds_bytes, s>>>(p);
+    const dim3 grid((unsigned)(pl.q_tiles * Hkv * pl.n_splits));
+    if (pl.rg == 1)
+        fa_prefill_kernel<1><<<grid, dim3(kThreads), lds_bytes, s>>>(p);
+    else
+        fa_prefill_kernel<2><<<grid, dim3(kThreads), lds_bytes, s>>>(p);
     profile_stop(prof, s);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_status(e, "fa_prefill launch");

@@ -255,6 +255,11 @@ def test_mask_form_start_chunk_costs_what_the_causal_form_does(sqa, orc, dev):
     (1280, 2000, 720, 16, 2),  # more than one round of workgroups per split
     (40, 1500, 0, 16, 2),      # rows that end far before the cache does: whole splits without a key
     (600, 600, 0, 4, 4),       # 128 positions per query tile
+    (8, 700, 692, 16, 2),      # 64 rows and
+    (9, 700, 691, 16, 2),      # 72: the two workgroup sizes
+    (512, 512, 0, 16, 2),      # an unsplit chunk in 64-row workgroups,
+    (30, 300, 270, 16, 1),     # four positions each,
+    (70, 300, 230, 4, 4),      # 64 positions each
 ])
 def test_prefill_split_plan(sqa, orc, dev, n_q, n_kv, q_pos0, H, Hkv):
     """Split counts, dispatch orders and merges of the plan, with the workspace
