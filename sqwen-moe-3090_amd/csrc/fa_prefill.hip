@@ -51,7 +51,7 @@
 // halves swapped when r & 8, and chunk c of Vc row d at c ^ ((d >> 1) & 3),
 // halves swapped when d & 8.
 //
-// Tiles move HBM -> LDS with global_load_lds_dwordx4: in iteration t the K half
+// Tiles move HBM -> LDS with global_load_lds_dwordx4, issued by the value waves: in iteration t the K half
 // (and mask rows) of tile t + 1 and the V half of tile t are in flight while
 // the score waves work on tile t and the value waves on tile t - 1; one
 // barrier per iteration.
@@ -563,24 +563,32 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         return;
     }
 
-    // ---------------- DMA: 1 KB per instruction, a fixed share per wave ---------
+    // ---------------- DMA: 1 KB per instruction, issued by the value waves --------
     // Iteration t: K half + mask of tile t + 1, V half of tile t (stage = tile & 1).
-    // K instruction jj (0..16, the last one 512 bytes) goes to wave jj % 8, V
-    // instruction jj to wave (jj + 4) % 8, mask instruction jm (< 8) to wave
-    // (jm + 2) % 8.
+    // K and V instructions jj (0..16, the last one 512 bytes) go to value wave jj %
+    // 4 and (jj + 2) % 4, mask instructions jm (< 8) to value waves (jm + 1) % 4: the
+    // score waves' chain is the longer one, they issue none (us per call, all waves
+    // issuing / this: 512 queries on 16896 keys 286 / 278.5, 2048 on 32048 1834 / 1807;
+    // raising the value waves' priority made the first 10% slower).
     const int n_mask_inst = p.mask ? (p.qb + 15) / 16 : 0;
     const uint8_t *kv_h = p.kv + (int64_t)kvh * p.kv_tiles * kTileBytes;
-    const int jk0 = wave, jv0 = (wave + 4) % kWaves, jm = (wave + kWaves - 2) % kWaves;
-    const bool has_m = jm < n_mask_inst;
-    static_assert(kKInst == 2 * kWaves + 1 && kVInst == 2 * kWaves + 1, "two full DMA instructions per wave and half");
-    const bool k_half = jk0 == 0, v_half = jv0 == 0;  // the wave that issues the 512-byte instruction
+    const int vw = wave & 3;
+    const int jv0 = (vw + 2) & 3;
+    static_assert(kKInst == 4 * kValueWaves + 1 && kVInst == 4 * kValueWaves + 1, "four full DMA instructions per value wave and half");
+    const bool k_half = vw == 0, v_half = jv0 == 0;  // the wave that issues the 512-byte instruction
     // mask row of this lane's slot in instruction jm: position q_base + r (clamped
     // to n_q - 1), chunk c = (s & 3) ^ ((r >> 1) & 3) of the row's 32 keys
-    const int m_r = (64 * jm + lane) >> 2;
-    const int m_c = ((64 * jm + lane) & 3) ^ ((m_r >> 1) & 3);
-    const uint32_t m_row =
-        has_m ? (uint32_t)((int64_t)(q_base + m_r < p.n_q ? q_base + m_r : p.n_q - 1) * p.mask_nb1) : 0u;
-    const bool m_lane = m_r < p.qb;
+    const int jm0 = (vw + 3) & 3;
+    uint32_t m_row[2];
+    int m_c[2];
+    bool m_lane[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int jm = jm0 + 4 * u, r = (64 * jm + lane) >> 2;
+        m_c[u] = ((64 * jm + lane) & 3) ^ ((r >> 1) & 3);
+        m_lane[u] = jm < n_mask_inst && r < p.qb;
+        m_row[u] = m_lane[u] ? (uint32_t)((int64_t)(q_base + r < p.n_q ? q_base + r : p.n_q - 1) * p.mask_nb1) : 0u;
+    }
     // record of the split's first tile (k_begin is a multiple of kPK); tile t's
     // record is t records further on
     const uint8_t *rec0 = kv_h + (k_begin / kPK) * kTileBytes;
@@ -588,26 +596,28 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         if (t_k >= 0) {
             const uint8_t *rec = rec0 + (int64_t)t_k * kTileBytes;
             const uint32_t st = lds0 + (uint32_t)((t_k & 1) * kKStage);
-            // instructions jk0 and jk0 + 8 (full), and 16 (512 bytes) on wave 0
-            dma16(1024u * jk0 + 16u * lane, rec, st + 1024u * jk0);
-            dma16(1024u * (jk0 + kWaves) + 16u * lane, rec, st + 1024u * (jk0 + kWaves));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dma16(1024u * (vw + 4 * r) + 16u * lane, rec, st + 1024u * (vw + 4 * r));
             if (k_half && lane < 32) dma16(1024u * (kKInst - 1) + 16u * lane, rec, st + 1024u * (kKInst - 1));
-            if (has_m) {
+            if (jm0 < n_mask_inst) {
                 const int64_t kt = k_begin + (int64_t)t_k * kPK;
-                const int64_t col = kt + 8 * m_c < p.mask_len ? kt + 8 * m_c : p.mask_len - 8;
-                const uint32_t sm = lds0 + (uint32_t)(kLdsMask + (t_k & 1) * p.mask_stage + 1024 * jm);
-                if (m_lane) dma16(m_row + (uint32_t)(2 * col), p.mask, sm);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int64_t col = kt + 8 * m_c[u] < p.mask_len ? kt + 8 * m_c[u] : p.mask_len - 8;
+                    const uint32_t sm = lds0 + (uint32_t)(kLdsMask + (t_k & 1) * p.mask_stage + 1024 * (jm0 + 4 * u));
+                    if (m_lane[u]) dma16(m_row[u] + (uint32_t)(2 * col), p.mask, sm);
+                }
             }
         }
         if (t_v >= 0) {
             const uint8_t *rec = rec0 + (int64_t)t_v * kTileBytes + kKHalf;
             const uint32_t st = lds0 + (uint32_t)(kLdsV + (t_v & 1) * kVStage);
-            dma16(1024u * jv0 + 16u * lane, rec, st + 1024u * jv0);
-            dma16(1024u * (jv0 + kWaves) + 16u * lane, rec, st + 1024u * (jv0 + kWaves));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dma16(1024u * (jv0 + 4 * r) + 16u * lane, rec, st + 1024u * (jv0 + 4 * r));
             if (v_half && lane < 32) dma16(1024u * (kVInst - 1) + 16u * lane, rec, st + 1024u * (kVInst - 1));
         }
     };
-    if (n_tiles > 0) issue(0, -1);
+    if (n_tiles > 0 && wave >= kScoreWaves) issue(0, -1);
 
     // the head's largest |d_v| over its 64-key groups, by every wavefront for itself
     uint32_t dv = 0;
@@ -704,10 +714,9 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         const int p_off = w * (kRG * 2048) + 16 * lane;  // P slots [w][rg][half][lane]
 
         for (int t = 0; t <= n_tiles && n_tiles > 0; ++t) {
-            // this wave's DMAs landed; the barrier makes every wave's visible and
-            // retires the buffers the new DMAs overwrite
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            issue(t + 1 < n_tiles ? t + 1 : -1, t < n_tiles ? t : -1);
+            // the value waves wait for their DMAs before this barrier, which makes them
+            // visible and retires the buffers the new ones overwrite
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             if (t == n_tiles) break;
             const int64_t kt = k_begin + (int64_t)t * kPK;
             const int nvalid = (int)(k_end - kt < kPK ? k_end - kt : kPK);
