@@ -3,7 +3,7 @@
 // src/model/attn.rs:228-251 in the reference (n_q = 512 or 2048 over a q4_0
 // cache of 16K-133K keys).
 //
-// Two short pre-passes, then one MFMA kernel:
+// Two short pre-passes in one launch, then one MFMA kernel:
 //   kvprep K, V q4_0 -> per 32-key tile and KV head: Kc fp16 codes (nib - 8)
 //                 [32 keys][256] and Dk fp16 scales [8 blocks][32 keys]; Vc
 //                 fp16 codes [256 dims][32 keys] and Dv fp16 scales [8 blocks]
@@ -51,10 +51,10 @@
 // halves swapped when r & 8, and chunk c of Vc row d at c ^ ((d >> 1) & 3),
 // halves swapped when d & 8.
 //
-// Tiles move HBM -> LDS with global_load_lds_dwordx4, issued by the value waves: in iteration t the K half
-// (and mask rows) of tile t + 1 and the V half of tile t are in flight while
-// the score waves work on tile t and the value waves on tile t - 1; one
-// barrier per iteration.
+// Tiles move HBM -> LDS with global_load_lds_dwordx4, issued by the value waves: in
+// iteration t the K half (and mask rows) of tile t + 1 and the V half of tile t
+// are in flight while the score waves work on tile t and the value waves on tile
+// t - 1; one barrier per iteration.
 //
 // Operand layout of the 16x16x32 MFMAs (64 lanes, lane = 16*g + n):
 //   A: A[row n][k = 8g..8g+7]   B: B[k = 8g..8g+7][col n]   C: C[rows 4g..4g+3][col n]
