@@ -66,8 +66,11 @@ __global__ __launch_bounds__(256) void fa_combine_kernel(const float *__restrict
     float o = 0.0f, l = 0.0f;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-        const float w = (M == -INFINITY || ml[j].x == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((ml[j].x - M) * kLog2e);
-        o = fmaf(acc[j], w, o);
+        // a prefill split in which the row sees no key (m = -inf) has left its acc
+        // unwritten: whatever the workspace holds there (0 * NaN) must not enter
+        const bool dead = ml[j].x == -INFINITY;
+        const float w = dead ? 0.0f : __builtin_amdgcn_exp2f((ml[j].x - M) * kLog2e);
+        o = dead ? o : fmaf(acc[j], w, o);
         l = fmaf(ml[j].y, w, l);
     }
     o += lane_xor16(o);

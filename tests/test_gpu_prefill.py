@@ -260,6 +260,14 @@ def test_mask_form_start_chunk_costs_what_the_causal_form_does(sqa, orc, dev):
     (512, 512, 0, 16, 2),      # an unsplit chunk in 64-row workgroups,
     (30, 300, 270, 16, 1),     # four positions each,
     (70, 300, 230, 4, 4),      # 64 positions each
+    (3, 768, 545, 16, 2),      # fewer than 256 rows and splits without a key: the padding
+    (5, 768, 600, 16, 2),      # of a cache to 256 rows,
+    (8, 1024, 762, 16, 2),
+    (8, 3072, 2820, 16, 2),
+    (15, 20224, 20011, 16, 2),
+    (15, 1500, 0, 16, 2),      # most of a cache,
+    (37, 1024, 700, 4, 4),     # a query group of one,
+    (31, 513, 482, 8, 1),      # and the second query tile's keys
 ])
 def test_prefill_split_plan(sqa, orc, dev, n_q, n_kv, q_pos0, H, Hkv):
     """Split counts, dispatch orders and merges of the plan, with the workspace
