@@ -18,10 +18,13 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/sqattn.h"
+#include "call.hpp"
 
 namespace {
 
-struct General {};  // leave the call to the Python wrapper
+using sqa_py::answer;
+using sqa_py::General;
+using sqa_py::without_gil;
 
 const at::Tensor &tensor(PyObject *o) {
     if (!THPVariable_CheckExact(o)) throw General();
@@ -108,25 +111,6 @@ sqa_tensor mask_view(const at::Tensor &m) {
 
 void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
-// Runs f (descriptors, then the library call under a released GIL) and returns
-// its status, or None for the general path
-template <class F>
-PyObject *answer(F f) {
-    int rc;
-    try {
-        rc = f();
-    } catch (...) {  // General, or torch refusing (the wrapper meets the same and reports it)
-        PyErr_Clear();
-        Py_RETURN_NONE;
-    }
-    return PyLong_FromLong(rc);
-}
-
-struct NoGil {
-    PyThreadState *s = PyEval_SaveThread();
-    ~NoGil() { PyEval_RestoreThread(s); }
-};
-
 // q, k_cache, v_cache, n_kv, mask, scale, max_bias, softcap, out, workspace
 PyObject *fa(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return answer([&]() -> int {
@@ -141,8 +125,9 @@ PyObject *fa(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const float scale = scale_of(a[5], q), bias = (float)real(a[6]), cap = (float)real(a[7]);
         void *wp = ws.data_ptr(), *st = stream();
         const size_t wb = (size_t)ws.numel();
-        NoGil g;
-        return sqa_flash_attn_ext(&tq, &tk, &tv, mask ? &tm : nullptr, scale, bias, cap, &to, wp, wb, st);
+        return without_gil([&] {
+            return sqa_flash_attn_ext(&tq, &tk, &tv, mask ? &tm : nullptr, scale, bias, cap, &to, wp, wb, st);
+        });
     });
 }
 
@@ -165,8 +150,9 @@ PyObject *fa_causal(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const float scale = scale_of(a[6], q);
         void *wp = ws.data_ptr(), *st = stream();
         const size_t wb = (size_t)ws.numel();
-        NoGil g;
-        return sqa_flash_attn_ext_causal(&tq, &tk, &tv, pos0, gate ? &tg : nullptr, scale, &to, wp, wb, st);
+        return without_gil([&] {
+            return sqa_flash_attn_ext_causal(&tq, &tk, &tv, pos0, gate ? &tg : nullptr, scale, &to, wp, wb, st);
+        });
     });
 }
 
@@ -177,8 +163,7 @@ PyObject *fill_mask(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const sqa_tensor tm = mask_view(tensor(a[0]));
         const int64_t start = integer(a[1]);
         void *st = stream();
-        NoGil g;
-        return sqa_fill_causal_mask(&tm, start, st);
+        return without_gil([&] { return sqa_fill_causal_mask(&tm, start, st); });
     });
 }
 
@@ -192,8 +177,7 @@ PyObject *set_rows(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const sqa_tensor td = cache_rows(tensor(a[0]), ne0), ts = rows2(src, ne0, src.size(0)),
                          ti = index(idx, SQA_TYPE_I64, idx.stride(0) * 8);
         void *st = stream();
-        NoGil g;
-        return sqa_set_rows_q4_0(&td, &ts, &ti, st);
+        return without_gil([&] { return sqa_set_rows_q4_0(&td, &ts, &ti, st); });
     });
 }
 
@@ -217,14 +201,14 @@ PyObject *rope_norm(PyObject *, PyObject *const *a, Py_ssize_t n) {
         void *st = stream();
         if (a[6] == Py_None) {
             const sqa_tensor to = make(SQA_TYPE_F32, dst, D, n_head, n_tok, 4, D * 4, n_head * D * 4, n_head * D * 4 * n_tok);
-            NoGil g;
-            return sqa_rope_norm_f32(&to, &ts, norm ? &tw : nullptr, eps, &tp, rope, st);
+            return without_gil([&] { return sqa_rope_norm_f32(&to, &ts, norm ? &tw : nullptr, eps, &tp, rope, st); });
         }
         const at::Tensor &idx = tensor(a[6]);
         need(idx.dim() >= 1);
         const sqa_tensor td = cache_rows(dst, n_head * D), ti = index(idx, SQA_TYPE_I64, idx.stride(0) * 8);
-        NoGil g;
-        return sqa_rope_norm_set_rows_q4_0(&td, &ts, norm ? &tw : nullptr, eps, &tp, rope, &ti, st);
+        return without_gil([&] {
+            return sqa_rope_norm_set_rows_q4_0(&td, &ts, norm ? &tw : nullptr, eps, &tp, rope, &ti, st);
+        });
     });
     if (view.obj) PyBuffer_Release(&view);
     return r;
@@ -247,8 +231,7 @@ PyObject *out_proj(PyObject *, PyObject *const *a, Py_ssize_t n) {
         }
         void *wp = ws.data_ptr(), *st = stream();
         const size_t wb = (size_t)ws.numel();
-        NoGil g;
-        return sqa_out_proj(&tw, &tx, gate ? &tg : nullptr, &to, wp, wb, st);
+        return without_gil([&] { return sqa_out_proj(&tw, &tx, gate ? &tg : nullptr, &to, wp, wb, st); });
     });
 }
 
@@ -265,8 +248,7 @@ PyObject *append(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const sqa_tensor tk = rows2(k, ne0, n_tok), tv = rows2(v, ne0, n_tok),
                          ti = make(SQA_TYPE_I64, tensor(a[4]), n_tok, 1, 1, 8, 8 * n_tok, 8 * n_tok, 8 * n_tok);
         void *st = stream();
-        NoGil g;
-        return sqa_kv_cache_append(kv, (int32_t)slot, &tk, &tv, &ti, st);
+        return without_gil([&] { return sqa_kv_cache_append(kv, (int32_t)slot, &tk, &tv, &ti, st); });
     });
 }
 
