@@ -204,7 +204,7 @@ int launch_rope_norm(const sqa_tensor *dst, const sqa_tensor &src, const sqa_ten
     p.theta_scale = theta_scale;
     p.freq_scale = rope.freq_scale;
     p.attn_factor = rope.attn_factor;
-    if (p.n_tok == 0) return SQA_OK;
+    if (p.n_tok == 0 || p.n_head == 0) return SQA_OK;
     const bool vec = (uintptr_t)src.data % 16 == 0 && src.nb[1] % 16 == 0 && src.nb[2] % 16 == 0;
     const bool q4 = idx != nullptr;
     if (q4) {

@@ -14,6 +14,8 @@ values but the extreme one, a code step away. Hence for the q4_0 output: |d|
 (fp16) equal or one ulp apart, at least 99.9% of the codes equal, every
 dequantised value within one code step of the oracle's, and rows outside idx
 untouched. The quantizer itself is bit-exact (test_gpu_set_rows.py)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -150,3 +152,20 @@ def test_heads_over_workgroups(sqa, dev, n_tok, n_head):
     for h in range(n_head):
         one = src[:, h:h + 1].contiguous()
         assert torch.equal(got[:, h:h + 1], sqa.rope_norm_f32(torch.zeros_like(one), one, w, 1e-6, pos, rope))
+
+
+def test_no_heads_is_no_work(sqa, dev):
+    """Tokens of zero heads are accepted and write nothing, in both forms."""
+    buf = torch.ones(1024, device=dev)
+    idx = torch.zeros(3, dtype=torch.int64, device=dev)
+    pos = torch.zeros(12, dtype=torch.int32, device=dev)
+    make, L = sqa.Tensor.make, sqa.lib()
+    src = make(sqa.TYPE_F32, [256, 0, 3], [4, 1024, 0], buf.data_ptr())
+    tp = make(sqa.TYPE_I32, [12], [4], pos.data_ptr())
+    ti = make(sqa.TYPE_I64, [3], [8], idx.data_ptr())
+    q4 = make(sqa.TYPE_Q4_0, [0, 4], [18, 0], buf.data_ptr())
+    rope = sqa.rope_params(64, (11, 11, 10, 0), 1e7)
+    r = ctypes.byref
+    assert L.sqa_rope_norm_f32(r(src), r(src), None, 1e-6, r(tp), r(rope), None) == 0
+    assert L.sqa_rope_norm_set_rows_q4_0(r(q4), r(src), None, 1e-6, r(tp), r(rope), r(ti), None) == 0
+    assert bool((buf == 1).all())
