@@ -260,7 +260,7 @@ def rope_norm_set_rows_q4_0(cache, src, norm_w, eps, pos, rope, idx, stream=None
     cache: uint8 (rows, ..., n_head*D//32*18) contiguous; src: float32 (n_tok, n_head, D)
     with contiguous rows; norm_w: float32 (D,) or None; pos: int32 (4*n_tok,);
     idx: int64 (n_tok,)."""
-    if stream is None and idx is not None:
+    if stream is None and idx is not None and isinstance(rope, Rope):
         rc = (_host or _load_host()).rope_norm(cache, src, norm_w, eps, pos, rope, idx)
         if rc is not None:
             if rc:
@@ -280,7 +280,7 @@ def rope_norm_set_rows_q4_0(cache, src, norm_w, eps, pos, rope, idx, stream=None
 
 def rope_norm_f32(out, src, norm_w, eps, pos, rope, stream=None):
     """Q producer (reference attn.rs:166-199): out float32 (n_tok, n_head, D) contiguous."""
-    if stream is None:
+    if stream is None and isinstance(rope, Rope):
         rc = (_host or _load_host()).rope_norm(out, src, norm_w, eps, pos, rope, None)
         if rc is not None:
             if rc:

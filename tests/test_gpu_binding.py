@@ -105,3 +105,14 @@ def test_refusals_are_the_wrappers(sqa, dev, gen):
                                                 sqa.rope_params(64, (11, 11, 10, 0), 1e7)), sqa.SqaError)):
         with pytest.raises(exc):
             bad()
+
+
+def test_rope_of_another_type_is_refused(sqa, dev):
+    src = torch.randn((1, 2, D), device=dev)
+    pos = torch.zeros(4, dtype=torch.int32, device=dev)
+    idx = torch.zeros(1, dtype=torch.int64, device=dev)
+    raw = bytes(sqa.rope_params(64, (11, 11, 10, 0), 1e7))  # the right bytes in the wrong object
+    with pytest.raises(TypeError):
+        sqa.rope_norm_f32(torch.empty_like(src), src, None, 1e-6, pos, raw)
+    with pytest.raises(TypeError):
+        sqa.rope_norm_set_rows_q4_0(torch.zeros((4, 2, RB), dtype=torch.uint8, device=dev), src, None, 1e-6, pos, raw, idx)
