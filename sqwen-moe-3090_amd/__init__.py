@@ -4,9 +4,9 @@ Python host mirror of the C ABI in include/sqattn.h, named after the ggml ops
 and the engine objects it stands in for (reference: src/backend/ffi.rs:363-405,
 src/engine/kv.rs). Device memory and streams come from PyTorch; every kernel
 runs from libsqattn.so, which sits next to this file. If the library is
-missing the import fails: there is no CPU fallback. Calls that give their output
-and workspace and use the current stream go through _sqahost.so
-(binding/host.cpp), the others build their descriptors here.
+missing the first call fails: there is no CPU fallback. Calls that give their
+output and workspace and use the current stream go through _sqahost.so
+(binding/host.cpp) where it was built, the others build their descriptors here.
 
 Tensor conventions (torch shapes, C order, all on the GPU):
   q       float32 (n_q, H, D)             the engine's [D, H, n_q] Q
@@ -155,12 +155,22 @@ def lib():
 _host = None
 
 
+class _General:
+    """Stands in for the native binding where it was not built: leaves every call
+    to the ctypes path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _load_host():
-    """The native binding of the hot entry points (raises if it was never built)."""
+    """The native binding of the hot entry points. A build without torch's headers
+    has none; one that is there has to load."""
     global _host
     lib()  # the binding links against the library beside it
     if not os.path.exists(HOST_PATH):
-        raise RuntimeError(f"{HOST_PATH} is missing: run __graft_entry__.build() first")
+        _host = _General()
+        return _host
     loader = importlib.machinery.ExtensionFileLoader("_sqahost", HOST_PATH)
     mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_sqahost", loader))
     loader.exec_module(mod)

@@ -1,5 +1,6 @@
 """Compile the HIP/C++ sources of this package into libsqattn.so for gfx950, and
-the Python binding of its hot entry points into _sqahost.so.
+the Python binding of its hot entry points into _sqahost.so (where the headers of
+torch and Python are there).
 
 Every source of csrc/ is compiled by hipcc (-x hip) into _build/, then linked
 into a shared library next to this file; binding/host.cpp is host code against
@@ -61,10 +62,20 @@ def _run(cmd, what):
         raise RuntimeError(f"{what} failed:\n" + r.stderr)
 
 
-def _compile_host(out):
-    import torch
-
+def _torch_root():
+    """torch's folder, or None where its C++ headers or Python's are missing (the
+    package then runs without the binding, every call on the ctypes path)."""
+    try:
+        import torch
+    except ImportError:
+        return None
     root = os.path.dirname(torch.__file__)
+    headers = (os.path.join(root, "include", "torch", "csrc", "autograd", "python_variable.h"),
+               os.path.join(sysconfig.get_paths()["include"], "Python.h"))
+    return root if all(os.path.exists(h) for h in headers) else None
+
+
+def _compile_host(root, out):
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
            sysconfig.get_paths()["include"], os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")]
     _run([HIPCC, "-std=c++17", "-O2", "-fPIC", "-Wall", "-x", "c++", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
@@ -78,21 +89,24 @@ def build(verbose=False):
     os.makedirs(bdir, exist_ok=True)
     srcs = sources()
     outs = [os.path.join(bdir, os.path.basename(s) + ".o") for s in srcs]
-    host = os.path.join(bdir, "host.o")
+    host, torch_root = os.path.join(bdir, "host.o"), _torch_root()
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
-        host_libs = ex.submit(_compile_host, host)
+        host_libs = ex.submit(_compile_host, torch_root, host) if torch_root else None
         list(ex.map(_compile, srcs, outs))
-        host_libs = host_libs.result()
+        host_libs = host_libs.result() if host_libs else None
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + outs, "link")
     os.replace(tmp, LIB)
-    # finds libsqattn.so beside itself; torch's libraries are loaded with torch
-    tmp = HOST + ".tmp"
-    _run([HIPCC, "-shared", "-fPIC", "-o", tmp, host, f"-L{HERE}", "-l:libsqattn.so", "-Wl,-rpath,$ORIGIN"] + host_libs,
-         "link of the binding")
-    os.replace(tmp, HOST)
+    if host_libs:
+        # finds libsqattn.so beside itself; torch's libraries are loaded with torch
+        tmp = HOST + ".tmp"
+        _run([HIPCC, "-shared", "-fPIC", "-o", tmp, host, f"-L{HERE}", "-l:libsqattn.so", "-Wl,-rpath,$ORIGIN"]
+             + host_libs, "link of the binding")
+        os.replace(tmp, HOST)
+    elif os.path.exists(HOST):
+        os.remove(HOST)  # of an earlier build, against an older library
     if verbose:
-        print("built", LIB, HOST)
+        print("built", LIB, HOST if host_libs else "(no headers of torch or Python: no native binding)")
     return LIB
 
 

@@ -188,3 +188,21 @@ def test_producer_argument_checks_before_any_launch(sqa):
     assert L.sqa_supports_rope_norm(by(out), by(src), None, by(pos), by(good), None) == 1
     assert L.sqa_supports_rope_norm(by(out), by(src), by(w), by(pos), by(sqa.rope_params(12, (3, 3, 0, 0), 1e7)),
                                     None) == 0
+
+
+def test_calls_without_the_native_binding(sqa, monkeypatch, tmp_path):
+    """Without _sqahost.so beside the library every call takes the ctypes path."""
+    import torch
+
+    monkeypatch.setattr(sqa, "_host", None)
+    monkeypatch.setattr(sqa, "HOST_PATH", str(tmp_path / "_sqahost.so"))
+    monkeypatch.setattr(sqa, "_stream", lambda stream: None)
+    mask = torch.zeros((2, 256), dtype=torch.float16)
+    for _ in range(2):  # the library's own refusal: reached, and again
+        with pytest.raises(sqa.SqaError) as e:
+            sqa.fill_causal_mask(mask, -1)
+        assert e.value.status == 6
+    (tmp_path / "_sqahost.so").write_bytes(b"not a library")  # one that is there has to load
+    monkeypatch.setattr(sqa, "_host", None)
+    with pytest.raises(ImportError):
+        sqa.fill_causal_mask(mask, -1)
