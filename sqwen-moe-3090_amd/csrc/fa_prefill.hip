@@ -1068,13 +1068,11 @@ int64_t max_splits(int64_t n_kv, int64_t wgs) {
 //   600 on 20600               610  432  426
 //   405 on 171568             4390 2331
 //   1280 on 6280               401  297  293
-//   2048 on 2048               145  145  128 (2 splits)
 constexpr float kWgTiles = 2.0f, kMergeTiles = 2.0f, kMergeRow = 1.2e-4f, kMargin = 0.98f;
 float tile_time(float busy) { return 0.75f + 0.25f * busy; }  // busy: share of the CUs
-bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
-int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q_tiles, int64_t rows) {
+int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q_tiles, int64_t rows, int64_t most) {
     const int64_t cus = device_cu_count(), wgs = q_tiles * Hkv;
-    const int64_t tiles = (n_kv + kPK - 1) / kPK, most = max_splits(n_kv, wgs);
+    const int64_t tiles = (n_kv + kPK - 1) / kPK;
     // key tiles that query tile i sees: first + i * step, at most all
     const float step = (float)qb / kPK;
     const float first = ((float)(n_kv > n_q ? n_kv - n_q : 0) + (float)qb) / kPK;
@@ -1118,6 +1116,77 @@ int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q
     return best_len * kPK;
 }
 
+// The same for a chunk whose query tiles see ranges of very different length (its
+// workgroups go out longest first, see the kernel), by walking through the dispatch:
+// workgroups are dealt strictly in turn to the XCDs and, inside one, in order and in
+// turn to its shader engines. One that finds its engine's CUs taken waits, and all
+// behind it with it, while CUs of the other engines are free; the dead workgroups of
+// a split take their turns. With that, 512 times of 64 causal chunks (300 to 2048
+// queries on 300 to 7169 keys, 1 to 8 splits, 16 heads on 2 or 4, 8 on 1) are met to
+// 2.3% RMS; with CUs taken as they come free inside an XCD to 4.4%. In tiles of 1.78
+// us. us per call with the estimate above, which takes dead workgroups as gone, with
+// this one, and with the best count of 1 to 12:
+//   768 queries on 768 keys     55.5  43.2  43.2 (before either 51.7)
+//   1500 on 1951               126.8 107.2 107.2
+//   1500 on 3001               180.4 157.2 157.2
+//   2000 on 2000, 4 KV heads   129.0 112.9 112.9
+//   600 on 1201, 8 heads on 1   49.0  36.0  36.0
+//   1300 on 1700, 4 on 4        54.9  41.7  41.7
+//   800 on 800, 4 on 4          35.7  34.8  30.8 (9 splits)
+// kSkewMany, more than 8 splits: 240 queries on 600 keys (8 on 2) 29.0 with 7, 30.3
+// with 10; 1400 on 1400 (4 on 4) 37.8 with 8, 40.6 with 9; 214 on 560 (4 on 4) 27.2
+// with 6, 25.6 with 9.
+// Host time 1 to 8 us.
+bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
+constexpr int kXcds = 8, kEngines = 4, kMaxEngineCus = 16;
+constexpr float kSkewWg = 5.0f, kSkewDead = 0.5f, kSkewMerge = 3.3f, kSkewRow = 0.85e-4f, kSkewMany = 0.6f;
+constexpr int64_t kSkewFew = 8;  // splits up to which a wavefront merges a row by itself
+int64_t split_skewed(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q_tiles, int64_t rows, int64_t most) {
+    // at most kMaxRounds * CUs workgroups where there is a choice, and n_kv < 4 n_q
+    const int wgs = (int)(q_tiles * Hkv), tiles = (int)((n_kv + kPK - 1) / kPK), hkv = (int)Hkv;
+    if (most <= 1) return (int64_t)tiles * kPK;
+    // keys up to the end of the last query tile, were it whole
+    const int ends = (int)((n_kv > n_q ? n_kv - n_q : 0) + q_tiles * qb), rows_qb = (int)qb;
+    int cus = device_cu_count() / (kXcds * kEngines);  // of an engine
+    cus = cus < 1 ? 1 : (cus > kMaxEngineCus ? kMaxEngineCus : cus);
+    int best_len = tiles, last_len = 0;
+    float best = INFINITY;
+    for (int s = 1; s <= (int)most; ++s) {
+        const int len = (tiles + s - 1) / s;
+        if (len == last_len) continue;
+        last_len = len;
+        const int n_s = (tiles + len - 1) / len, total = n_s * wgs;
+        // unsplit must not only tie: kMargin
+        const float first = (float)len + kSkewWg;
+        const float merge = n_s == 1 ? (kMargin - 1.0f) * first
+                                     : kSkewMerge + kSkewRow * (float)(n_s * rows) + (n_s > kSkewFew ? kSkewMany : 0.0f);
+        float end = first;  // of the last workgroup; that of the first one at least
+        for (int x : {0, kXcds - 1}) {  // the first and the last XCD stand for all
+            if (end + merge >= best) break;
+            float at[kEngines][kMaxEngineCus], now = 0.0f;  // a CU is busy up to here; the time of the dispatch
+            int r = x, from = 0, e = 0, c = 0;              // place in its split, the split's first tile; engine, CU
+            for (int i = x; i < total; i += kXcds, r += kXcds) {
+                for (; r >= wgs; r -= wgs) from += len;
+                // tiles up to the last query of its query tile, inside the split
+                const int keys = ends - r / hkv * rows_qb;
+                const int sees = (keys < (int)n_kv ? (keys + kPK - 1) / kPK : tiles) - from;
+                const float busy = sees > 0 ? (float)(sees < len ? sees : len) + kSkewWg : kSkewDead;
+                float *cu = &at[e][c];
+                if (c == cus) {  // all taken once: the one that is free first
+                    cu = at[e];
+                    for (int j = 1; j < cus; ++j) cu = at[e][j] < *cu ? &at[e][j] : cu;
+                    now = *cu > now ? *cu : now;
+                }
+                *cu = now + busy;
+                end = *cu > end ? *cu : end;
+                if (++e == kEngines) e = 0, c += c < cus;
+            }
+        }
+        if (end + merge < best) best = end + merge, best_len = len;
+    }
+    return (int64_t)best_len * kPK;
+}
+
 PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     PrefillPlan pl{};
     const int G = (int)(H / Hkv);
@@ -1133,11 +1202,13 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     pl.mask_stage = pl.qb * kPK * 2;
     pl.kv_tiles = (n_kv + 63) / 64 * 2;  // the pre-pass writes 64-key groups
     pl.q_tiles = (int)((n_q + pl.qb - 1) / pl.qb);
-    pl.split_len = split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H);
+    const int64_t most = max_splits(n_kv, pl.q_tiles * Hkv);
+    pl.split_len = skewed(n_q, n_kv) ? split_skewed(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most)
+                                     : split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most);
     pl.n_splits = (int)((n_kv + pl.split_len - 1) / pl.split_len);
     // partials: for the most splits that a cache of up to n_kv keys can get, so
     // that a workspace sized for a longer cache serves every shorter one
-    const int64_t parts = max_splits(n_kv, pl.q_tiles * Hkv);
+    const int64_t parts = most;
     size_t o = 0;
     pl.off_kv = o; o = al256(o + (size_t)Hkv * pl.kv_tiles * kTileBytes);
     pl.off_dvmax = o; o = al256(o + (size_t)Hkv * (size_t)(pl.kv_tiles / 2) * 4);

@@ -286,3 +286,29 @@ def test_prefill_split_plan(sqa, orc, dev, n_q, n_kv, q_pos0, H, Hkv):
         err = rel_err(got.cpu().numpy()[rows], ref)
         print(f"split plan {form} n_q={n_q} n_kv={n_kv} at {q_pos0}: max err / rms = {err:.3e}")
         assert err <= TOL
+
+
+@pytest.mark.parametrize("small,large,H,Hkv", [(768, 900, 16, 2), (752, 900, 16, 4)])
+def test_a_smaller_first_chunk_takes_no_longer(sqa, orc, dev, small, large, H, Hkv):
+    """The split count of a causal chunk has to be chosen with the workgroups that
+    see no key in mind (one split too many: 55 us for 768 first queries, 48 for 900)."""
+    calls = []
+    for n in (small, large):
+        q, kq, vq = qkv(orc, n, n, n, H=H, Hkv=Hkv)
+        qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(x)).to(dev) for x in (q, kq, vq))
+        out = torch.empty((n, H, 256), device=dev)
+        ws = torch.empty(sqa.flash_attn_workspace_size(qd, kd, n), dtype=torch.uint8, device=dev)
+        calls.append(lambda a=(qd, kd, vd, n, 0), o=out, w=ws: sqa.flash_attn_ext_causal(*a, out=o, workspace=w))
+    times = [[], []]
+    for r in range(9):
+        for i in ((0, 1) if r % 2 == 0 else (1, 0)):
+            t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            t0.record()
+            for _ in range(20):
+                calls[i]()
+            t1.record()
+            torch.cuda.synchronize()
+            times[i].append(t0.elapsed_time(t1) / 20 * 1e3)
+    a, b = (sorted(t)[4] for t in times)
+    print(f"{small} first queries: {a:.1f} us, {large}: {b:.1f} us")
+    assert a <= 1.03 * b
