@@ -170,8 +170,12 @@ int sqa_flash_attn_ext(const sqa_tensor *q, const sqa_tensor *k, const sqa_tenso
                        const sqa_tensor *dst, void *workspace, size_t workspace_bytes,
                        void *stream);
 
-/* Workspace bytes sqa_flash_attn_ext / sqa_flash_attn_ext_causal need for
- * these shapes (0 is a valid answer). */
+/* Workspace bytes sqa_flash_attn_ext / sqa_flash_attn_ext_causal use for
+ * these shapes (0 is a valid answer). Of a prefill chunk they grow with n_kv, so a
+ * workspace sized for the longest cache serves every shorter one; they do not
+ * always grow with n_q (fewer queries are split over more key ranges). A prefill
+ * chunk in a smaller workspace takes fewer splits of its keys, and is refused with
+ * SQA_ERR_WORKSPACE only where one round of splits does not fit. */
 size_t sqa_flash_attn_ext_workspace_size(const sqa_tensor *q, const sqa_tensor *k,
                                          const sqa_tensor *v, const sqa_tensor *dst);
 

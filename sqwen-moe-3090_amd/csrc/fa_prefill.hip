@@ -1022,31 +1022,54 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
     }
 }
 
-size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
-
 struct PrefillPlan {
     int64_t kv_tiles;
-    int rg, qb, q_tiles, n_splits, mask_stage;
-    int64_t split_len;
-    size_t off_kv, off_dvmax, off_qh, off_ql, off_mask, off_lim, off_pa, off_pm, total;
+    int rg, qb, q_tiles, mask_stage;
+    int64_t most, least;  // key splits: that the plan may choose; that a workspace has to hold
+    size_t off_kv, off_dvmax, off_qh, off_ql, off_mask, off_lim, off_pa, total;
 };
 
-// Key splits of a chunk. A workgroup fills a CU (LDS), so the workgroups of one
-// split (wgs = q_tiles per KV head) run in rounds of one per CU. Up to an eighth
-// of the CUs, whole splits fill a round to 8/9 or more; with more workgroups
-// per split, up to kMaxRounds rounds let a later one fill what a single round
-// leaves idle (160 workgroups: 2 rounds of 3 splits instead of 2 of 2).
+size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Bytes of the split partials of `rows` rows: O [n_splits][rows][256], then (m, l)
+size_t partial_acc_bytes(int64_t n_splits, int64_t rows) { return al256((size_t)(n_splits * rows) * kHeadDim * 4); }
+size_t partial_bytes(int64_t n_splits, int64_t rows) {
+    return n_splits > 1 ? partial_acc_bytes(n_splits, rows) + al256((size_t)(n_splits * rows) * 8) : 0;
+}
+
+// Key splits that are worth a try. A workgroup fills a CU (LDS), so the workgroups
+// of one split (wgs = q_tiles per KV head) run in rounds of one per CU. Up to an
+// eighth of the CUs, whole splits fill a round to 8/9 or more. With more workgroups
+// per split, the fewest splits that fill their rounds best, of up to kMaxRounds
+// rounds: 160 workgroups run 2 rounds of 3 splits, where one or two splits leave
+// 3/8 of each round idle; 64 run one round of 4, and no more fill it better (us per
+// call with the count that 4 rounds would allow and the estimate then takes / with
+// this one: 1233 queries on 5303 keys 315 / 248, 1345 on 8800 (4 KV heads) 474 / 438,
+// 1555 on 9975 (8 heads on 1) 355 / 278). A skewed chunk, half of whose workgroups
+// may see no key, is tried up to twice the splits that one round takes.
 // Up to kOneSplitKeys keys a chunk stays whole: its output and gate leave in the
 // attention kernel's epilogue, with no partials and no merge.
 constexpr int kMinSplitTiles = 2;  // 64 keys
 constexpr int kMaxRounds = 4;
 constexpr int kOneSplitKeys = 512;
-int64_t max_splits(int64_t n_kv, int64_t wgs) {
+bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
+int64_t max_splits(int64_t n_kv, int64_t wgs, bool skew) {
     if (n_kv <= kOneSplitKeys) return 1;
     const int64_t cus = device_cu_count();
     const int64_t by_len = ((n_kv + kPK - 1) / kPK + kMinSplitTiles - 1) / kMinSplitTiles;
-    const int64_t by_rounds = (8 * wgs > cus ? kMaxRounds : 1) * cus / wgs;
-    int64_t s = by_len < by_rounds ? by_len : by_rounds;
+    int64_t s = cus / wgs;
+    if (8 * wgs > cus) {
+        const int64_t rounds = kMaxRounds * cus / wgs;
+        float best = 0.0f;
+        s = 1;
+        for (int64_t i = 1; i <= rounds; ++i) {
+            const float fill = (float)(i * wgs) / (float)((i * wgs + cus - 1) / cus * cus);
+            if (fill > 1.01f * best) best = fill, s = i;
+        }
+        const int64_t tries = (cus + wgs - 1) / wgs * 2;
+        if (skew && tries > s) s = tries < rounds ? tries : rounds;
+    }
+    if (s > by_len) s = by_len;
     if (s > kMaxSplits) s = kMaxSplits;
     return s < 1 ? 1 : s;
 }
@@ -1132,14 +1155,16 @@ int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q
 //   2000 on 2000, 4 KV heads   129.0 112.9 112.9
 //   600 on 1201, 8 heads on 1   49.0  36.0  36.0
 //   1300 on 1700, 4 on 4        54.9  41.7  41.7
-//   800 on 800, 4 on 4          35.7  34.8  30.8 (9 splits)
-// kSkewMany, more than 8 splits: 240 queries on 600 keys (8 on 2) 29.0 with 7, 30.3
-// with 10; 1400 on 1400 (4 on 4) 37.8 with 8, 40.6 with 9; 214 on 560 (4 on 4) 27.2
-// with 6, 25.6 with 9.
-// Host time 1 to 8 us.
-bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
+//   800 on 800, 4 on 4          35.7  34.8  30.8 (9 splits; kSkewMany: 245 on 576,
+//   8 on 2, 28.7 with 6 splits and 30.7 with 9)
+// Over 142 random shapes (132 to 2048 queries, 1 to 8 KV heads, every count up to 16)
+// its choice costs 0.4% more than the best count on average, 5% of the shapes lose
+// more than 3%; with the estimate above it was 3.2% and 25%. Host time 1 to 5 us.
 constexpr int kXcds = 8, kEngines = 4, kMaxEngineCus = 16;
 constexpr float kSkewWg = 5.0f, kSkewDead = 0.5f, kSkewMerge = 3.3f, kSkewRow = 0.85e-4f, kSkewMany = 0.6f;
+// a split chunk has to be clearly ahead of an unsplit one, and a second round of a
+// first one (2000 queries on 4001 keys, 8 on 1: 135 us with 2 splits, 142 with 5)
+constexpr float kSkewMargin = 0.96f, kSkewLate = 1.04f;
 constexpr int64_t kSkewFew = 8;  // splits up to which a wavefront merges a row by itself
 int64_t split_skewed(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q_tiles, int64_t rows, int64_t most) {
     // at most kMaxRounds * CUs workgroups where there is a choice, and n_kv < 4 n_q
@@ -1156,21 +1181,21 @@ int64_t split_skewed(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t
         if (len == last_len) continue;
         last_len = len;
         const int n_s = (tiles + len - 1) / len, total = n_s * wgs;
-        // unsplit must not only tie: kMargin
         const float first = (float)len + kSkewWg;
-        const float merge = n_s == 1 ? (kMargin - 1.0f) * first
+        const float merge = n_s == 1 ? (kSkewMargin - 1.0f) * first
                                      : kSkewMerge + kSkewRow * (float)(n_s * rows) + (n_s > kSkewFew ? kSkewMany : 0.0f);
-        float end = first;  // of the last workgroup; that of the first one at least
-        for (int x : {0, kXcds - 1}) {  // the first and the last XCD stand for all
+        float end = first, late = 1.0f;  // of the last workgroup; that of the first one at least
+        for (int x : {0, kXcds / 2}) {  // two XCDs stand for all (the same picks)
             if (end + merge >= best) break;
             float at[kEngines][kMaxEngineCus], now = 0.0f;  // a CU is busy up to here; the time of the dispatch
-            int r = x, from = 0, e = 0, c = 0;              // place in its split, the split's first tile; engine, CU
+            int r = x, from = 0, e = 0, c = 0, live = 0;    // place in its split, the split's first tile; engine, CU
             for (int i = x; i < total; i += kXcds, r += kXcds) {
                 for (; r >= wgs; r -= wgs) from += len;
                 // tiles up to the last query of its query tile, inside the split
                 const int keys = ends - r / hkv * rows_qb;
                 const int sees = (keys < (int)n_kv ? (keys + kPK - 1) / kPK : tiles) - from;
                 const float busy = sees > 0 ? (float)(sees < len ? sees : len) + kSkewWg : kSkewDead;
+                live += sees > 0;
                 float *cu = &at[e][c];
                 if (c == cus) {  // all taken once: the one that is free first
                     cu = at[e];
@@ -1181,7 +1206,9 @@ int64_t split_skewed(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t
                 end = *cu > end ? *cu : end;
                 if (++e == kEngines) e = 0, c += c < cus;
             }
+            if (live > cus * kEngines) late = kSkewLate;
         }
+        end *= late;
         if (end + merge < best) best = end + merge, best_len = len;
     }
     return (int64_t)best_len * kPK;
@@ -1202,13 +1229,12 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     pl.mask_stage = pl.qb * kPK * 2;
     pl.kv_tiles = (n_kv + 63) / 64 * 2;  // the pre-pass writes 64-key groups
     pl.q_tiles = (int)((n_q + pl.qb - 1) / pl.qb);
-    const int64_t most = max_splits(n_kv, pl.q_tiles * Hkv);
-    pl.split_len = skewed(n_q, n_kv) ? split_skewed(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most)
-                                     : split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most);
-    pl.n_splits = (int)((n_kv + pl.split_len - 1) / pl.split_len);
-    // partials: for the most splits that a cache of up to n_kv keys can get, so
-    // that a workspace sized for a longer cache serves every shorter one
-    const int64_t parts = most;
+    const int64_t wgs = pl.q_tiles * Hkv, rows = n_q * H;
+    pl.most = max_splits(n_kv, wgs, skewed(n_q, n_kv));
+    // one round of splits of 512 keys or more
+    pl.least = (cus + wgs - 1) / wgs;
+    if (pl.least > (n_kv + 511) / 512) pl.least = (n_kv + 511) / 512;
+    if (pl.least > pl.most) pl.least = pl.most;
     size_t o = 0;
     pl.off_kv = o; o = al256(o + (size_t)Hkv * pl.kv_tiles * kTileBytes);
     pl.off_dvmax = o; o = al256(o + (size_t)Hkv * (size_t)(pl.kv_tiles / 2) * 4);
@@ -1217,20 +1243,30 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     pl.off_mask = o; o = al256(o + (size_t)n_q * ((n_kv + 7) / 8 * 8) * 2);
     pl.off_lim = o; o = al256(o + (size_t)pl.q_tiles * 4);
     pl.off_pa = o;
-    pl.off_pm = o;
-    if (parts > 1) {
-        o = al256(o + (size_t)parts * n_q * H * kHeadDim * 4);
-        pl.off_pm = o;
-        o = al256(o + (size_t)parts * n_q * H * 2 * 4);
-    }
-    pl.total = o + 256;
+    pl.total = o + partial_bytes(pl.most, rows) + 256;
     return pl;
+}
+
+// A workspace sized for a longer cache serves every shorter one: the layout before
+// the partials grows with n_kv, the splits of a chunk that is not skewed do, and
+// those of skewed chunks are all asked for by the longest of them.
+size_t plan_bytes(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
+    const size_t here = plan(n_q, H, Hkv, n_kv).total;
+    if (skewed(n_q, n_kv)) return here;
+    const size_t skew = plan(n_q, H, Hkv, 4 * n_q - 1).total;
+    return here > skew ? here : skew;
+}
+
+// Keys per split with partials of at most `most` splits
+int64_t split_len(const PrefillPlan &pl, int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv, int64_t most) {
+    return skewed(n_q, n_kv) ? split_skewed(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most)
+                             : split_keys(n_q, n_kv, Hkv, pl.qb, pl.q_tiles, n_q * H, most);
 }
 
 }  // namespace
 
 size_t fa_prefill_workspace(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
-    return plan(n_q, H, Hkv, n_kv).total;
+    return plan_bytes(n_q, H, Hkv, n_kv);
 }
 
 int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
@@ -1239,9 +1275,16 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     const int G = (int)(H / Hkv);
     if (16 % G != 0) return set_error(SQA_ERR_UNSUPPORTED, "prefill: n_head/n_head_kv must divide 16");
     const PrefillPlan pl = plan(n_q, H, Hkv, n_kv);
-    if (!a.ws || a.ws_bytes < pl.total)
-        return set_error(SQA_ERR_WORKSPACE, "flash_attn_ext: workspace %zu bytes < %zu needed", a.ws_bytes,
-                         pl.total);
+    // A workspace sized for another shape may hold fewer partials than the plan would
+    // use (the size is not monotone in n_q): the chunk then takes fewer splits.
+    const int64_t rows = n_q * H;
+    const size_t need = pl.off_pa + partial_bytes(pl.least, rows) + 256;
+    if (!a.ws || a.ws_bytes < need)
+        return set_error(SQA_ERR_WORKSPACE, "flash_attn_ext: workspace %zu bytes < %zu needed", a.ws_bytes, need);
+    int64_t most = pl.most;
+    while (a.ws_bytes < pl.off_pa + partial_bytes(most, rows) + 256) --most;  // down to pl.least
+    const int64_t len = split_len(pl, n_q, H, Hkv, n_kv, most);
+    const int n_splits = (int)((n_kv + len - 1) / len);
     uint8_t *base = reinterpret_cast<uint8_t *>(((uintptr_t)a.ws + 255) & ~(uintptr_t)255);
     uint8_t *kv = base + pl.off_kv;
     uint32_t *dvmax = reinterpret_cast<uint32_t *>(base + pl.off_dvmax);
@@ -1315,16 +1358,16 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     p.G = G;
     p.Hkv = (int)Hkv;
     p.q_pos0 = a.q_pos0;
-    p.n_splits = pl.n_splits;
+    p.n_splits = n_splits;
     p.q_tiles = pl.q_tiles;
-    p.split_len = pl.split_len;
+    p.split_len = len;
     p.skew = skewed(n_q, n_kv);
     p.qb = pl.qb;
     p.mask_stage = pl.mask_stage;
     p.part_acc = reinterpret_cast<float *>(base + pl.off_pa);
-    p.part_ml = reinterpret_cast<float *>(base + pl.off_pm);
+    p.part_ml = reinterpret_cast<float *>(base + pl.off_pa + partial_acc_bytes(n_splits, rows));
     p.dst = (float *)a.dst->data;
-    p.gate = (pl.n_splits == 1 && a.gate) ? (const char *)a.gate->data : nullptr;
+    p.gate = (n_splits == 1 && a.gate) ? (const char *)a.gate->data : nullptr;
     p.gate_nb1 = a.gate ? (int64_t)a.gate->nb[1] : 0;
     p.gate_nb2 = a.gate ? (int64_t)a.gate->nb[2] : 0;
 
@@ -1342,7 +1385,7 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     });
     if (lds_err != hipSuccess) return hip_status(lds_err, "fa_prefill LDS attribute");
     prof = profile_start("fa_prefill", s);
-    const dim3 grid((unsigned)(pl.q_tiles * Hkv * pl.n_splits));
+    const dim3 grid((unsigned)(pl.q_tiles * Hkv * n_splits));
     if (pl.rg == 1)
         fa_prefill_kernel<1><<<grid, dim3(kThreads), lds_bytes, s>>>(p);
     else
@@ -1350,8 +1393,8 @@ int launch_fa_prefill(const FaArgs &a, hipStream_t s) {
     profile_stop(prof, s);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_status(e, "fa_prefill launch");
-    if (pl.n_splits > 1)
-        return launch_fa_combine(p.part_acc, p.part_ml, pl.n_splits, (int)(n_q * H), p.dst, a.gate, (int)H, s);
+    if (n_splits > 1)
+        return launch_fa_combine(p.part_acc, p.part_ml, n_splits, (int)rows, p.dst, a.gate, (int)H, s);
     return SQA_OK;
 }
 

@@ -100,8 +100,20 @@ def test_prefill_workspace_of_a_longer_cache_serves_a_shorter_one(sqa, n_q):
     for n_kv in list(range(32, 4096, 96)) + [8192, 20048, 65536, 65568, 172032]:
         q, k, o = fa_descs(sqa, n_q=n_q, n_kv=n_kv)
         need = L.sqa_flash_attn_ext_workspace_size(ctypes.byref(q), ctypes.byref(k), ctypes.byref(k), ctypes.byref(o))
-        assert need >= last > -1
+        assert need >= last and need > 0
         last = need
+
+
+@pytest.mark.parametrize("n_q,n_kv,splits", [(512, 16896, 6), (300, 3328, 20), (2048, 133120, 1), (37, 20224, 42),
+                                             (1280, 6400, 4)])
+def test_prefill_workspace_holds_what_the_plan_uses(sqa, n_q, n_kv, splits):
+    """Tile records, Q pairs and a mask copy, and partials for the splits that the
+    plan may choose, not for every count that four rounds of workgroups could take."""
+    q, k, o = fa_descs(sqa, n_q=n_q, n_kv=n_kv)
+    need = sqa.lib().sqa_flash_attn_ext_workspace_size(ctypes.byref(q), ctypes.byref(k), ctypes.byref(k), ctypes.byref(o))
+    rows = n_q * 16
+    bare = 2 * (n_kv // 32) * 33792 + rows * 256 * 4 + n_q * n_kv * 2
+    assert bare < need <= bare + (splits * rows * 258 * 4 if splits > 1 else 0) + (1 << 16)
 
 
 class FakeKv:

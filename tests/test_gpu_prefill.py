@@ -312,3 +312,21 @@ def test_a_smaller_first_chunk_takes_no_longer(sqa, orc, dev, small, large, H, H
     a, b = (sorted(t)[4] for t in times)
     print(f"{small} first queries: {a:.1f} us, {large}: {b:.1f} us")
     assert a <= 1.03 * b
+
+
+@pytest.mark.parametrize("n_q,sized_for,n_kv", [(512, 640, 8192), (600, 640, 8192), (300, 512, 3328), (40, 48, 1500)])
+def test_workspace_of_another_chunk_size(sqa, orc, dev, n_q, sized_for, n_kv):
+    """One workspace, sized for the largest chunk, serves the smaller ones, with fewer
+    splits where it holds fewer partials than their own size asks for."""
+    q, kq, vq = qkv(orc, n_q + n_kv, n_q, n_kv)
+    rows = np.unique(np.r_[0:n_q:max(1, n_q // 6), n_q - 1])
+    pos = n_kv - n_q
+    ref = np.concatenate([orc.flash_attn_ext_causal(q[r:r + 1], kq, vq, pos + int(r)) for r in rows])
+    qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(x)).to(dev) for x in (q, kq, vq))
+    size = sqa.flash_attn_workspace_size(torch.empty((sized_for, 16, 256), device=dev), kd, n_kv)
+    ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=dev)
+    got = sqa.flash_attn_ext_causal(qd, kd, vd, n_kv, pos, workspace=ws)
+    assert rel_err(got.cpu().numpy()[rows], ref) <= TOL
+    with pytest.raises(sqa.SqaError) as e:  # what cannot hold one round of splits is refused
+        sqa.flash_attn_ext_causal(qd, kd, vd, n_kv, pos, workspace=ws[:2 * (n_kv // 32) * 33792])
+    assert e.value.status == 3
