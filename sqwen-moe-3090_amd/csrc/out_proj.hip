@@ -45,10 +45,13 @@ __device__ __forceinline__ float h2f(uint32_t bits) {
 }
 
 // ---------------------------------------------------------------- op_prep
-// One wavefront per (16 tokens, 64 values of K): lane 16q + n takes values 8q ..
-// 8q + 7 of both 32-value sub-blocks of token n and writes xg = x *
-// sigmoid(gate) as fp16 hi and lo in the order in which op_gemm reads them, 1 KB
-// per load. B operand (c, e) of super-block s, c < 4, e < 2, holds in lane 16g + n
+// One wavefront per (16 tokens, 32-value sub-block of K): lane 16q + n takes values
+// 8q .. 8q + 7 of token n and writes xg = x * sigmoid(gate) as fp16 hi and lo in the
+// order in which op_gemm reads them, 1 KB per load. Its time is one chain of load, exp
+// and store; a wavefront per two sub-blocks leaves half as many to overlap: us per
+// call of the whole projection, that / this: 33 tokens, N = 5120, K = 2048 17.3 / 14.6,
+// 100, 8192, 2048 20.1 / 19.2, 300, 4096, 4096 46.6 / 46.0, 512, 2048, 4096 34.0 / 33.7.
+// B operand (c, e) of super-block s, c < 4, e < 2, holds in lane 16g + n
 // the values 64g + 32e + 8c .. + 7 of token n: an MFMA then takes from each lane
 // group another code group (64 values, 32 bytes of a weight row), so a lane needs
 // 32 consecutive weight bytes and two of the 8 scales. hi and lo of tile T at
@@ -69,77 +72,74 @@ __device__ __forceinline__ float xsum32(float x) {
 template <bool GATE, bool VEC>
 __global__ __launch_bounds__(256) void op_prep_kernel(const char *__restrict__ x, int64_t x_nb1,
                                                       const char *__restrict__ gate, int64_t g_nb1, int K, int M,
-                                                      int tiles, uint4 *__restrict__ xb, uint4 *__restrict__ sb) {
+                                                      int tiles, uint4 *__restrict__ xb, uint16_t *__restrict__ sb) {
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int kp = K / 64;  // sub-block pairs
+    const int subs = K / 32;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wid >= (int64_t)tiles * kp) return;
-    const int T = (int)(wid / kp), pr = (int)(wid - (int64_t)T * kp);
+    if (wid >= (int64_t)tiles * subs) return;
+    const int T = (int)(wid / subs), sub = (int)(wid - (int64_t)T * subs);
+    const int pr = sub >> 1, e = sub & 1;  // sub-block pair (64 values), which of the two
     const int t = 16 * T + n;
-    uint32_t sw[2][3];  // the three parts of S of both sub-blocks
+    float v[8], gv[8];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        float v[8], gv[8];
+    for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
+    if (t < M) {
+        const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 32 * sub + 8 * g;
+        const float *gr = GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 32 * sub + 8 * g : nullptr;
+        if (VEC) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
-        if (t < M) {
-            const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 64 * pr + 32 * e + 8 * g;
-            const float *gr =
-                GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 64 * pr + 32 * e + 8 * g : nullptr;
-            if (VEC) {
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const float4 a = reinterpret_cast<const float4 *>(xr)[c];
-                    v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
-                    if (GATE) {
-                        const float4 b = reinterpret_cast<const float4 *>(gr)[c];
-                        gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    v[j] = xr[j];
-                    if (GATE) gv[j] = gr[j];
+            for (int c = 0; c < 2; ++c) {
+                const float4 a = reinterpret_cast<const float4 *>(xr)[c];
+                v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
+                if (GATE) {
+                    const float4 b = reinterpret_cast<const float4 *>(gr)[c];
+                    gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
                 }
             }
-            if (GATE) {
+        } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
+            for (int j = 0; j < 8; ++j) {
+                v[j] = xr[j];
+                if (GATE) gv[j] = gr[j];
             }
         }
-        float sum = 0.0f;
-        uint16_t hb[8], lb[8];
+        if (GATE) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            sum += v[j];
-            float a = v[j];
-            // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
-            asm volatile("" : "+v"(a));
-            const _Float16 h = (_Float16)a;
-            const _Float16 l = (_Float16)(a - (float)h);
-            __builtin_memcpy(&hb[j], &h, 2);
-            __builtin_memcpy(&lb[j], &l, 2);
+            for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
         }
-        uint4 a, b;
-        __builtin_memcpy(&a, hb, 16);
-        __builtin_memcpy(&b, lb, 16);
-        uint4 *o = xb + ((int64_t)T * (2 * kp) + 8 * (pr >> 2) + 2 * g + e) * 128 + 16 * (pr & 3) + n;
-        o[0] = a;
-        o[64] = b;
-        // S = its leading 8 bits (truncated) + those of the rest, twice: each
-        // difference is exact
-        float r = xsum32(xsum16(sum));
+    }
+    float sum = 0.0f;
+    uint16_t hb[8], lb[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        sum += v[j];
+        float a = v[j];
+        // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
+        asm volatile("" : "+v"(a));
+        const _Float16 h = (_Float16)a;
+        const _Float16 l = (_Float16)(a - (float)h);
+        __builtin_memcpy(&hb[j], &h, 2);
+        __builtin_memcpy(&lb[j], &l, 2);
+    }
+    uint4 a, b;
+    __builtin_memcpy(&a, hb, 16);
+    __builtin_memcpy(&b, lb, 16);
+    uint4 *o = xb + ((int64_t)T * subs + 8 * (pr >> 2) + 2 * g + e) * 128 + 16 * (pr & 3) + n;
+    o[0] = a;
+    o[64] = b;
+    // S = its leading 8 bits (truncated) + those of the rest, twice: each
+    // difference is exact
+    float r = xsum32(xsum16(sum));
+    if (g == (pr & 3)) {
+        uint16_t *s = sb + (((int64_t)T * (subs / 8) + (pr >> 2)) * 64 + lane) * 8 + e;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const uint32_t top = __float_as_uint(r) & 0xFFFF0000u;
-            sw[e][c] = top >> 16;
+            s[2 * c] = (uint16_t)(top >> 16);
             r -= __uint_as_float(top);
         }
+        s[6] = 0;
     }
-    if (g == (pr & 3))
-        sb[((int64_t)T * (kp / 4) + (pr >> 2)) * 64 + lane] =
-            make_uint4(sw[0][0] | (sw[1][0] << 16), sw[0][1] | (sw[1][1] << 16), sw[0][2] | (sw[1][2] << 16), 0u);
 }
 
 // ---------------------------------------------------------------- op_gemm
@@ -750,7 +750,8 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     if (!ws || ws_bytes < need)
         return set_error(SQA_ERR_WORKSPACE, "out_proj: workspace %zu bytes < %zu needed", ws_bytes, need);
     uint8_t *base = reinterpret_cast<uint8_t *>(((uintptr_t)ws + 255) & ~(uintptr_t)255);
-    uint4 *xb = reinterpret_cast<uint4 *>(base), *sb = reinterpret_cast<uint4 *>(base + L.sb);
+    uint4 *xb = reinterpret_cast<uint4 *>(base);
+    uint16_t *sb = reinterpret_cast<uint16_t *>(base + L.sb);
     static std::once_flag g2_once;
     static hipError_t g2_err = hipSuccess;
     std::call_once(g2_once, [] {
@@ -761,7 +762,7 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     const int prof = profile_start("out_proj", s);
     const bool vec = (uintptr_t)x.data % 16 == 0 && x.nb[1] % 16 == 0 &&
                      (!gate || ((uintptr_t)gate->data % 16 == 0 && gate->nb[1] % 16 == 0));
-    const dim3 pg((unsigned)((L.tiles * (K / 64) + 3) / 4));
+    const dim3 pg((unsigned)((L.tiles * (K / 32) + 3) / 4));
     const char *xd = (const char *)x.data, *gd = gate ? (const char *)gate->data : nullptr;
     const int64_t xn = (int64_t)x.nb[1], gn = gate ? (int64_t)gate->nb[1] : 0;
     const int Ki = (int)K, Mi = (int)M, tl = (int)L.tiles;
@@ -777,7 +778,7 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     p.w = (const uint8_t *)w.data;
     p.w_nb1 = (int64_t)w.nb[1];
     p.xb = xb;
-    p.sb = sb;
+    p.sb = reinterpret_cast<const uint4 *>(sb);
     p.K = Ki;
     p.N = (int)N;
     p.M = Mi;
