@@ -207,23 +207,30 @@ __device__ __forceinline__ void op_scale_add(const OpHead &h, int g, const float
     }
 }
 
-// Workgroups go round-robin to the 8 XCDs: the id of workgroup lin such that each
-// XCD takes a contiguous run of ids, i.e. of token tiles (every row block of
-// them), and its L2 serves their operands to all their row blocks.
-__device__ __forceinline__ int xcd_order(int lin, int nb) {
-    const int x = lin & 7, per = nb >> 3, rem = nb & 7;
-    return x * per + (x < rem ? x : rem) + (lin >> 3);
-}
-
 struct GemmParams {
     const uint8_t *w;
     int64_t w_nb1;
     const uint4 *xb, *sb;  // B operands, see op_prep
     int K, N, M, tiles;    // tiles of 16 tokens
-    int row_blocks;        // workgroups along N
+    int row_blocks, token_groups;  // workgroups along N, along the tokens
+    bool rows_first;       // order of the workgroups, see place_of
     float *dst;
     int64_t d_nb1;
 };
+
+// Workgroups go round-robin to the 8 XCDs: the row block and token group of
+// workgroup lin such that each XCD takes a contiguous run of them, either of token
+// groups (every row block of them: its L2 then serves their operands to all row
+// blocks, and all XCDs read all weights) or, with rows_first, of row blocks.
+struct Place {
+    int row_block, token_group;
+};
+__device__ __forceinline__ Place place_of(const GemmParams &p) {
+    const int lin = (int)blockIdx.x, nb = (int)gridDim.x;
+    const int x = lin & 7, per = nb >> 3, rem = nb & 7;
+    const int id = x * per + (x < rem ? x : rem) + (lin >> 3);
+    return p.rows_first ? Place{id / p.token_groups, id % p.token_groups} : Place{id % p.row_blocks, id / p.row_blocks};
+}
 
 // A workgroup of KS wavefronts owns 16 RT rows of W and 16 TT tokens; wavefront w
 // takes super-blocks w, w + KS, ... of K, reading weights and operands straight
@@ -245,9 +252,9 @@ __global__ __launch_bounds__(64 * KS) void op_gemm_kernel(GemmParams p) {
     __shared__ float red[KS][RT * TT][4][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int id = xcd_order((int)blockIdx.x, (int)gridDim.x);
-    const int r0 = (id % p.row_blocks) * 16 * RT;
-    const int T0 = (id / p.row_blocks) * TT;
+    const Place at = place_of(p);
+    const int r0 = at.row_block * 16 * RT;
+    const int T0 = at.token_group * TT;
     const int nsb = p.K / kQK;
 
     floatx4 acc[RT][TT];
@@ -390,9 +397,9 @@ __global__ __launch_bounds__(64 * kG2Waves) void op_gemm2_kernel(GemmParams p) {
     uint8_t(*ss)[kG2SBytes] = reinterpret_cast<uint8_t(*)[kG2SBytes]>(lds + 2 * (kG2Half + kG2WBytes));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int id = xcd_order((int)blockIdx.x, (int)gridDim.x);
-    const int row0 = (id % p.row_blocks) * kG2Rows;
-    const int T0 = (id / p.row_blocks) * TT;
+    const Place at = place_of(p);
+    const int row0 = at.row_block * kG2Rows;
+    const int T0 = at.token_group * TT;
     const int nsb = p.K / kQK;
     const uint32_t xs0 = (uint32_t)(uintptr_t)&xs[0][0], wb0 = (uint32_t)(uintptr_t)&wb[0][0];
     const uint32_t ss0 = (uint32_t)(uintptr_t)&ss[0][0];
@@ -785,11 +792,12 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     p.tiles = tl;
     p.dst = (float *)dst.data;
     p.d_nb1 = (int64_t)dst.nb[1];
-#define SQA_GEMM(KS, RT, TT)                                                                                \
-    do {                                                                                                    \
-        p.row_blocks = (int)((N + 16 * RT - 1) / (16 * RT));                                                \
-        op_gemm_kernel<KS, RT, TT><<<dim3((unsigned)(p.row_blocks * ((tl + TT - 1) / TT))), dim3(64 * KS), 0, \
-                                     s>>>(p);                                                              \
+    p.rows_first = false;
+#define SQA_GEMM(KS, RT, TT)                                                                                   \
+    do {                                                                                                       \
+        p.row_blocks = (int)((N + 16 * RT - 1) / (16 * RT));                                                   \
+        p.token_groups = (tl + TT - 1) / TT;                                                                   \
+        op_gemm_kernel<KS, RT, TT><<<dim3((unsigned)(p.row_blocks * p.token_groups)), dim3(64 * KS), 0, s>>>(p); \
     } while (0)
     // units of 16 rows x 16 tokens. Few of them: the smallest workgroup tile of
     // op_gemm that still leaves at most one workgroup per CU (with two the time
@@ -810,7 +818,15 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
         SQA_GEMM(8, 4, 2);
     } else {
         p.row_blocks = (int)((N + kG2Rows - 1) / kG2Rows);
-        op_gemm2_kernel<<<dim3((unsigned)(p.row_blocks * ((tl + kG2TT - 1) / kG2TT))), dim3(64 * kG2Waves), kG2Lds, s>>>(p);
+        p.token_groups = (tl + kG2TT - 1) / kG2TT;
+        // Every XCD reads all of one, weights or operands, and its share of the other:
+        // row blocks first where the weights are clearly the larger. us per call, token
+        // groups / row blocks first: 100 tokens, N = 8192, K = 2048 (weights 10 times the
+        // operands) 19.2 / 17.3, 200 of them 28.3 / 27.0, 300, 4096, 4096 (1.9) 46.1 / 44.1,
+        // 1000, 8192, 2048 (1.14) 100.8 / 102.6, 512, 2048, 4096 (0.56) 33.4 / 34.3.
+        // op_gemm's calls are all better with token groups first (128 tokens 13.8 / 15.5).
+        p.rows_first = 2 * (uint64_t)N * (K / kQK) * kBlockBytes > 3 * (uint64_t)L.sb;
+        op_gemm2_kernel<<<dim3((unsigned)(p.row_blocks * p.token_groups)), dim3(64 * kG2Waves), kG2Lds, s>>>(p);
     }
 #undef SQA_GEMM
     profile_stop(prof, s);

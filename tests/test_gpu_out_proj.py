@@ -118,3 +118,10 @@ def test_out_proj_tile_rule_edges(sqa, orc, dev, M, K):
     # of 16 rows x 16 tokens on 256 CUs), last token tiles full and ragged, one
     # super-block and 7 (fewer than and not a multiple of the K splits)
     assert run(sqa, orc, dev, 2048, K, M, 300 + M + K, outliers=4) <= TOL
+
+
+@pytest.mark.parametrize("M,N", [(70, 8208), (200, 4160), (600, 4160), (600, 1040)])
+def test_out_proj_workgroup_orders(sqa, orc, dev, M, N):
+    # row blocks first (weights larger than the operands) and token groups first, with
+    # a ragged last row block and numbers of workgroups that 8 does not divide
+    assert run(sqa, orc, dev, N, 512, M, 700 + M, outliers=4) <= TOL
