@@ -799,22 +799,28 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
         p.token_groups = (tl + TT - 1) / TT;                                                                   \
         op_gemm_kernel<KS, RT, TT><<<dim3((unsigned)(p.row_blocks * p.token_groups)), dim3(64 * KS), 0, s>>>(p); \
     } while (0)
-    // units of 16 rows x 16 tokens. Few of them: the smallest workgroup tile of
-    // op_gemm that still leaves at most one workgroup per CU (with two the time
-    // doubles); more: op_gemm2. us at N = 2048, K = 4096 with op_prep, op_gemm
-    // <16, 1, 1> / <16, 1, 2> / <16, 2, 2> / <8, 4, 2> / op_gemm2: 23 tokens 9.9 / 12.3 /
-    // 14.3 / 20.5 / 28.1, 64 tokens 13.8 / 13.0 / 14.4 / 20.5 / 28.2, 128 tokens 23.1 /
-    // 20.4 / 15.4 / 20.9 / 28.6, 256 tokens 39 / 36 / 27.6 / 23.6 / 30.6, 300 tokens 46 /
-    // 43 / 36 / 38 / 31.9, 512 tokens 70 / 62 / 46 / 41 / 32.8. op_gemm2's DMA
+    // The smallest workgroup tile of op_gemm that still leaves at most one workgroup
+    // per CU (with two the time grows by half or doubles), counted with the tokens and
+    // rows that fill a tile up; for one token tile also two per CU of the smallest, as the
+    // second tile of the others would be thrown away; else op_gemm2. us at N = 2048, K =
+    // 4096 with op_prep, op_gemm <16, 1, 1> / <16, 1, 2> / <16, 2, 2> / <8, 4, 2> /
+    // op_gemm2: 23 tokens 9.9 / 12.3 / 14.3 / 20.5 / 28.1, 64 tokens 13.8 / 13.0 / 14.4 /
+    // 20.5 / 28.2, 128 tokens 23.1 / 20.4 / 15.4 / 20.9 / 28.6, 256 tokens 39 / 36 / 27.6 /
+    // 23.6 / 30.6, 300 tokens 46 / 43 / 36 / 38 / 31.9, 512 tokens 70 / 62 / 46 / 41 / 32.8.
+    // K = 4096, <16, 1, 1> / <16, 1, 2> / <16, 2, 2> / <8, 4, 2>: 16 tokens, N = 5120 12.5 /
+    // 16.9 / 13.3 / 19.2, 48 tokens, 2720 13.0 / 18.2 / 13.9 / 20.0, 48 tokens, 5120 21.3 /
+    // 24.1 / 21.9 / 19.7. K does not enter: at K = 1024, where 12 of the 16 wavefronts have
+    // no super-block, 48 tokens with N = 2720 take 8.7 / 11.6 / 9.9 / 11.4. op_gemm2's DMA
     // addresses its 128 rows with 32-bit offsets.
-    const int64_t cus = device_cu_count(), units = N / 16 * L.tiles;
-    if (units <= cus) {
+    const int64_t cus = device_cu_count(), row_tiles = N / 16;
+    auto groups = [&](int64_t rt, int64_t tt) { return (row_tiles + rt - 1) / rt * ((L.tiles + tt - 1) / tt); };
+    if (groups(1, 1) <= (L.tiles == 1 ? 2 : 1) * cus) {
         SQA_GEMM(16, 1, 1);
-    } else if (units <= 2 * cus) {
+    } else if (groups(1, 2) <= cus) {
         SQA_GEMM(16, 1, 2);
-    } else if (units <= 4 * cus) {
+    } else if (groups(2, 2) <= cus) {
         SQA_GEMM(16, 2, 2);
-    } else if (units <= 8 * cus || (uint64_t)kG2Rows * w.nb[1] >= (1ull << 32)) {
+    } else if (groups(4, 2) <= cus || (uint64_t)kG2Rows * w.nb[1] >= (1ull << 32)) {
         SQA_GEMM(8, 4, 2);
     } else {
         p.row_blocks = (int)((N + kG2Rows - 1) / kG2Rows);

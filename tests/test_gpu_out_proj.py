@@ -125,3 +125,34 @@ def test_out_proj_workgroup_orders(sqa, orc, dev, M, N):
     # row blocks first (weights larger than the operands) and token groups first, with
     # a ragged last row block and numbers of workgroups that 8 does not divide
     assert run(sqa, orc, dev, N, 512, M, 700 + M, outliers=4) <= TOL
+
+
+@pytest.mark.parametrize("N,M", [(5120, 16), (8208, 16), (2720, 33), (2720, 48), (5120, 33), (4608, 100)])
+def test_out_proj_tile_rule_counts_workgroups(sqa, orc, dev, N, M):
+    # tiles that rows or tokens fill up only in part: one token tile at one, two and more
+    # workgroups per CU, three token tiles, a last row block of 32 rows
+    assert run(sqa, orc, dev, N, 512, M, 900 + M, outliers=4) <= TOL
+
+
+def test_fewer_tokens_take_no_longer(sqa, dev):
+    """One token tile on 5120 rows (two workgroups of 16 rows per CU at most) against two
+    token tiles: tiles that compute a token tile to throw it away took 17 us against 14."""
+    rng = np.random.default_rng(5)
+    w = torch.from_numpy(random_q4k(rng, 5120, 4096)).to(dev)
+    times, calls = [[], []], []
+    for M in (16, 32):
+        x, g, o = (torch.randn((M, n), device=dev) for n in (4096, 4096, 5120))
+        ws = torch.empty(sqa.out_proj_workspace_size(w, x), dtype=torch.uint8, device=dev)
+        calls.append(lambda x=x, g=g, o=o, ws=ws: sqa.out_proj(w, x, gate=g, out=o, workspace=ws))
+    for r in range(9):
+        for i in ((0, 1) if r % 2 == 0 else (1, 0)):
+            t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            t0.record()
+            for _ in range(50):
+                calls[i]()
+            t1.record()
+            torch.cuda.synchronize()
+            times[i].append(t0.elapsed_time(t1) / 50 * 1e3)
+    a, b = (sorted(t)[4] for t in times)
+    print(f"W_o, 5120 rows: 16 tokens {a:.1f} us, 32 tokens {b:.1f} us")
+    assert a <= 1.05 * b
