@@ -23,18 +23,40 @@ def gen(dev):
     return g
 
 
-def both(call, state):
-    """state before, bytes after the native call and after the Python one."""
+class Watch:
+    """The native binding, with a record of its answers (None: left to Python)."""
+
+    def __init__(self, host):
+        self.host, self.answers = host, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.answers.append(getattr(self.host, name)(*args))
+            return self.answers[-1]
+        return call
+
+
+@pytest.fixture(autouse=True)
+def watch(sqa, monkeypatch):
+    w = Watch(sqa._host or sqa._load_host())
+    monkeypatch.setattr(sqa, "_host", w)
+    return w
+
+
+def both(call, state, watch):
+    """Equal bytes from the native call, which has to answer, and from the Python one."""
     got = []
     for kw in ({}, {"stream": torch.cuda.current_stream()}):
         s = {k: v.clone() for k, v in state.items()}
+        watch.answers.clear()
         call(s, **kw)
+        assert watch.answers == ([] if kw else [0])
         got.append([v.cpu().numpy().tobytes() for v in s.values()])
     assert got[0] == got[1]
 
 
 @pytest.mark.parametrize("n_q,strided,masked", [(1, False, True), (1, True, False), (3, True, True), (40, True, True)])
-def test_attention_calls(sqa, dev, gen, n_q, strided, masked):
+def test_attention_calls(sqa, dev, gen, watch, n_q, strided, masked):
     n_kv = 768
     kc, vc = cache(gen, 1024, dev), cache(gen, 1024, dev)
     wide = torch.randn((n_q, 2 * H, D + 16), generator=gen, device=dev)
@@ -43,18 +65,18 @@ def test_attention_calls(sqa, dev, gen, n_q, strided, masked):
     mask = torch.zeros((n_q, 2 * n_kv), dtype=torch.float16, device=dev)[:, :n_kv] if masked else None
     if masked:
         both(lambda s, **kw: sqa.fill_causal_mask(s["mask"][:, :n_kv], 700, **kw),
-             {"mask": torch.zeros((n_q, 2 * n_kv), dtype=torch.float16, device=dev)})
+             {"mask": torch.zeros((n_q, 2 * n_kv), dtype=torch.float16, device=dev)}, watch)
         sqa.fill_causal_mask(mask, 700)
     ws = torch.empty(sqa.flash_attn_workspace_size(q, kc, n_kv), dtype=torch.uint8, device=dev)
     out = {"out": torch.zeros((n_q, H, D), device=dev)}
     for scale in (None, 0.05):
-        both(lambda s, **kw: sqa.flash_attn_ext(q, kc, vc, n_kv, mask=mask, scale=scale, out=s["out"], workspace=ws, **kw), out)
+        both(lambda s, **kw: sqa.flash_attn_ext(q, kc, vc, n_kv, mask=mask, scale=scale, out=s["out"], workspace=ws, **kw), out, watch)
         both(lambda s, **kw: sqa.flash_attn_ext_causal(q, kc, vc, n_kv, 700, gate=gate, scale=scale, out=s["out"],
-                                                       workspace=ws, **kw), out)
+                                                       workspace=ws, **kw), out, watch)
 
 
 @pytest.mark.parametrize("n,strided", [(1, False), (5, True)])
-def test_producer_cache_and_projection_calls(sqa, dev, gen, n, strided):
+def test_producer_cache_and_projection_calls(sqa, dev, gen, watch, n, strided):
     wide = torch.randn((n, 2 * H, D), generator=gen, device=dev)
     src = wide[:, ::2] if strided else wide[:, :H].contiguous()
     w = torch.rand(D, generator=gen, device=dev)
@@ -64,10 +86,10 @@ def test_producer_cache_and_projection_calls(sqa, dev, gen, n, strided):
     k = {"c": cache(gen, 64, dev)}
     for norm in (w, None):
         both(lambda s, **kw: sqa.rope_norm_f32(s["o"], src, norm, 1e-6, pos, rope, **kw),
-             {"o": torch.zeros((n, H, D), device=dev)})
-        both(lambda s, **kw: sqa.rope_norm_set_rows_q4_0(s["c"], src[:, :HKV], norm, 1e-6, pos, rope, idx, **kw), k)
+             {"o": torch.zeros((n, H, D), device=dev)}, watch)
+        both(lambda s, **kw: sqa.rope_norm_set_rows_q4_0(s["c"], src[:, :HKV], norm, 1e-6, pos, rope, idx, **kw), k, watch)
     both(lambda s, **kw: sqa.set_rows_q4_0(s["c"], src[:, 0].repeat(1, 2) if not strided else wide.view(n, -1)[:, 5:517],
-                                           idx, **kw), k)
+                                           idx, **kw), k, watch)
     wq = torch.randint(0, 256, (64, 4, 144), generator=gen, device=dev, dtype=torch.uint8)
     wq[..., 1], wq[..., 3] = 0x10, 0x10  # finite fp16 d and dmin
     wq = wq.view(64, 576)[::2] if strided else wq.view(64, 576)
@@ -75,7 +97,7 @@ def test_producer_cache_and_projection_calls(sqa, dev, gen, n, strided):
     ws = torch.empty(max(1, sqa.out_proj_workspace_size(wq, x)), dtype=torch.uint8, device=dev)
     for g in (gate, None):
         both(lambda s, **kw: sqa.out_proj(wq, x, gate=g, out=s["o"], workspace=ws, **kw),
-             {"o": torch.zeros((n, wq.shape[0]), device=dev)})
+             {"o": torch.zeros((n, wq.shape[0]), device=dev)}, watch)
 
     caches = []
     for kw in ({}, {"stream": torch.cuda.current_stream()}):
@@ -83,12 +105,14 @@ def test_producer_cache_and_projection_calls(sqa, dev, gen, n, strided):
         kv.zero_caches()
         kv.begin_step(n)
         rows = src[:, :HKV].reshape(n, -1).contiguous()
+        watch.answers.clear()
         kv.append(1, rows, -rows, torch.arange(n, device=dev), **kw)
+        assert watch.answers == ([] if kw else [0])
         caches.append([t.cpu().numpy() for t in kv.k + kv.v])
     assert all(np.array_equal(a, b) for a, b in zip(*caches)) and caches[0][1].any()
 
 
-def test_refusals_are_the_wrappers(sqa, dev, gen):
+def test_refusals_are_the_wrappers(sqa, dev, gen, watch):
     kc = cache(gen, 256, dev)
     q = torch.randn((1, H, D), generator=gen, device=dev)
     out, ws = torch.empty_like(q), torch.empty(sqa.flash_attn_workspace_size(q, kc, 256), dtype=torch.uint8, device=dev)
@@ -103,8 +127,11 @@ def test_refusals_are_the_wrappers(sqa, dev, gen):
                      (lambda: sqa.set_rows_q4_0(kc, q[0], torch.zeros(16, dtype=torch.int64, device=dev)), AssertionError),
                      (lambda: sqa.rope_norm_f32(out, q, None, 1e-6, torch.zeros(3, dtype=torch.int32, device=dev),
                                                 sqa.rope_params(64, (11, 11, 10, 0), 1e7)), sqa.SqaError)):
+        watch.answers.clear()
         with pytest.raises(exc):
             bad()
+        assert len(watch.answers) == 1 and watch.answers[0] != 0
+        assert exc is sqa.SqaError or watch.answers[0] is None
 
 
 def test_rope_of_another_type_is_refused(sqa, dev):
@@ -116,3 +143,24 @@ def test_rope_of_another_type_is_refused(sqa, dev):
         sqa.rope_norm_f32(torch.empty_like(src), src, None, 1e-6, pos, raw)
     with pytest.raises(TypeError):
         sqa.rope_norm_set_rows_q4_0(torch.zeros((4, 2, RB), dtype=torch.uint8, device=dev), src, None, 1e-6, pos, raw, idx)
+
+
+def test_calls_run_on_the_current_stream(sqa, dev, gen, watch):
+    """The native path and the Python one look the stream up by different routes: a
+    call inside torch.cuda.stream() has to wait for that stream's work."""
+    side = torch.cuda.Stream()
+    big, idx = torch.ones(1 << 26, device=dev), torch.arange(4, device=dev)
+    for n in (1, 2):  # the second time every kernel is loaded
+        src = torch.zeros((4, 512), device=dev)
+        want = torch.zeros((8, HKV, RB), dtype=torch.uint8, device=dev)
+        sqa.set_rows_q4_0(want, src + n, idx)
+        got = torch.zeros_like(want)
+        torch.cuda.synchronize()
+        watch.answers.clear()
+        with torch.cuda.stream(side):
+            for _ in range(40):
+                big.mul_(1.0)
+            src.fill_(n)
+            sqa.set_rows_q4_0(got, src, idx)
+        side.synchronize()
+        assert watch.answers == [0] and torch.equal(got, want)
