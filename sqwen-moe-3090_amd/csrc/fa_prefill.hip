@@ -19,7 +19,8 @@
 //
 // fa_prefill_kernel: a workgroup takes 128 (or 64) query rows of ONE KV head (GQA
 // packed: row r is position r / G, head kvh*G + r % G) and streams 32-key
-// tiles. Its 8 wavefronts (2 per SIMD) split the work by kind:
+// tiles. Its 8 wavefronts (2 per SIMD) split the work by kind (rows and registers
+// for 128 query rows, half of both for 64):
 //   score wave w (0..3), rows 32w..32w+31, holds their Q' hi and lo (128
 //     registers): S^T = sum over q4_0 blocks b of d_k[b] * (Kc_b.Q'h_b +
 //     Kc_b.Q'l_b), the products on v_mfma_f32_16x16x32_f16 (all exact in
@@ -85,9 +86,9 @@ constexpr int kVInst = (kVHalf + 1023) / 1024;  // 17, the last one 512 bytes
 constexpr int kKStage = kKInst * 1024, kVStage = kVInst * 1024;
 // LDS map (sized for kMaxRG): 2 K stages | 2 V stages | 2 P buffers | 2 rescale buffers | 2 mask stages
 constexpr int kLdsV = 2 * kKStage;
-constexpr int kLdsP = kLdsV + 2 * kVStage;        // [4 waves][2 rg][2 halves][64 lanes][16 B]
+constexpr int kLdsP = kLdsV + 2 * kVStage;        // [4 waves][kRG][2 halves][64 lanes][16 B]
 constexpr int kPBuf = kScoreWaves * kMaxRG * 2 * 1024;
-constexpr int kLdsA = kLdsP + 2 * kPBuf;          // [4 waves][2 rg][16 rows] f32
+constexpr int kLdsA = kLdsP + 2 * kPBuf;          // [4 waves][kRG][16 rows] f32
 constexpr int kABuf = kScoreWaves * kMaxRG * 16 * 4;
 constexpr int kLdsMask = kLdsA + 2 * kABuf;       // [qb positions][32 keys] f16
 constexpr float kLog2e = 1.4426950408889634f;
@@ -497,7 +498,7 @@ struct PrefillParams {
     int q_tiles;        // workgroups per (KV head, split)
     bool skew;          // order of the workgroups, see the kernel
     int64_t split_len;  // keys per split, a multiple of kPK
-    int qb;             // query positions per workgroup (128 / G)
+    int qb;             // query positions per workgroup (64 or 128 rows / G)
     int mask_stage;     // LDS bytes per mask stage (qb x 64)
     float *part_acc, *part_ml;  // n_splits > 1
     float *dst;                 // n_splits == 1: [n_q][H][256]
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
     if (wave < kScoreWaves) {
         const int w = wave;
         float *ml = reinterpret_cast<float *>(smem + kLdsP) + w * (kRG * 32);  // [rg][row][m, l]
-        // Q' hi and lo of rows r = 32w + 16rg + n (position q_base + r / G, head
+        // Q' hi and lo of rows r = 16 kRG w + 16rg + n (position q_base + r / G, head
         // kvh*G + r % G) as B operands, dims 32b + 8g..+7
         half8 bqh[kRG][8], bql[kRG][8];
         int my_pos[kRG], m_off[kRG];
@@ -897,7 +898,7 @@ __global__ __launch_bounds__(kThreads, 1) void fa_prefill_kernel(PrefillParams p
         return;
     }
 
-    // ---- value waves: O[row 32w + 16rg + 4g + i][dim 16T + n] ----------------
+    // ---- value waves: O[row 16 kRG w + 16rg + 4g + i][dim 16T + n] ----------------
     const int w = wave - kScoreWaves;
     const float *ml = reinterpret_cast<const float *>(smem + kLdsP) + w * (kRG * 32);  // [rg][row][m, l]
     // V operand of dim 16T + n, keys 8g..8g+7: chunk g ^ ((n >> 1) & 3), halves swapped when n & 8.
@@ -1048,7 +1049,13 @@ size_t partial_bytes(int64_t n_splits, int64_t rows) {
 // 1555 on 9975 (8 heads on 1) 355 / 278). A skewed chunk, half of whose workgroups
 // may see no key, is tried up to twice the splits that one round takes.
 // Up to kOneSplitKeys keys a chunk stays whole: its output and gate leave in the
-// attention kernel's epilogue, with no partials and no merge.
+// attention kernel's epilogue, with no partials and no merge. The line is a bound on
+// what a short context asks for, not where the forms cross: first chunks, us per call
+// whole in 64-row workgroups / in 128-row ones with the best split count: 448 queries
+// 30.0 / 33.2, 512 32.6 / 34.7, 544 34.0 / 36.5, 640 37.9 / 38.3, 768 42.8 / 42.9, 1024 52.1 /
+// 53.8 (with 2 or 3 splits of 64-row workgroups 28.8 at 512, 33.8 at 640), so the first
+// is taken up to the line and the second past it; and a few queries on a full 512 keys
+// walk 16 tiles in a row (8 queries 29.9, 19.9 on 768 keys in 64-key splits).
 constexpr int kMinSplitTiles = 2;  // 64 keys
 constexpr int kMaxRounds = 4;
 constexpr int kOneSplitKeys = 512;
@@ -1218,10 +1225,11 @@ PrefillPlan plan(int64_t n_q, int64_t H, int64_t Hkv, int64_t n_kv) {
     PrefillPlan pl{};
     const int G = (int)(H / Hkv);
     // 64-row workgroups where 128 rows would leave most of their work to padding or
-    // most of the chip idle: a query tile of all the rows, and an unsplit chunk
-    // whose 64-row workgroups still run in one round. A tile of keys costs them
-    // about 1.5 us where 128 rows take 2.2 to 2.4: us per call 128 rows / 64 rows 512
-    // first queries 48.3 / 35.1, 200 first queries 32.3 / 21.5, 8 on 3008 keys 34 / 24.
+    // most of the chip idle: a query tile of all the rows, and an unsplit chunk (for
+    // that line see max_splits) whose 64-row workgroups still run in one round. A tile
+    // of keys costs them about 1.5 us where 128 rows take 2.2 to 2.4: us per call 128
+    // rows / 64 rows 512 first queries 48.3 / 35.1, 200 first queries 32.3 / 21.5, 8 on
+    // 3008 keys 34 / 24.
     const int64_t cus = device_cu_count();
     const int64_t wgs64 = (n_q + rows_per_wg(1) / G - 1) / (rows_per_wg(1) / G) * Hkv;
     pl.rg = n_q * G <= rows_per_wg(1) || (n_kv <= kOneSplitKeys && wgs64 <= cus) ? 1 : 2;

@@ -16,9 +16,9 @@
 //             the sub-block sums S = sum xg as the B operand of the min term
 //   op_gemm   16x16x32 f16 MFMAs over the raw codes: every product exact, then d
 //             and dmin per super-block in fp32. Two forms by the amount of work:
-//             op_gemm (K split over the wavefronts, no barrier) while its tiles
-//             give a CU at most one workgroup, else op_gemm2 (operands shared
-//             through LDS)
+//             op_gemm (K split over the wavefronts, no barrier) while one of its
+//             tiles leaves a CU at most one workgroup, else op_gemm2 (operands
+//             shared through LDS)
 //
 // MFMA operand layouts (lane = 16*g + n):
 //   16x16x32 f16: A[n][8g..8g+7]   B[8g..8g+7][n]   C[4g..4g+3][n]
@@ -807,6 +807,7 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     // op_gemm2: 23 tokens 9.9 / 12.3 / 14.3 / 20.5 / 28.1, 64 tokens 13.8 / 13.0 / 14.4 /
     // 20.5 / 28.2, 128 tokens 23.1 / 20.4 / 15.4 / 20.9 / 28.6, 256 tokens 39 / 36 / 27.6 /
     // 23.6 / 30.6, 300 tokens 46 / 43 / 36 / 38 / 31.9, 512 tokens 70 / 62 / 46 / 41 / 32.8.
+    // (With a pre-pass 0.5 to 1 us slower than this one: 23 tokens are 9.1 now.)
     // K = 4096, <16, 1, 1> / <16, 1, 2> / <16, 2, 2> / <8, 4, 2>: 16 tokens, N = 5120 12.5 /
     // 16.9 / 13.3 / 19.2, 48 tokens, 2720 13.0 / 18.2 / 13.9 / 20.0, 48 tokens, 5120 21.3 /
     // 24.1 / 21.9 / 19.7. K does not enter: at K = 1024, where 12 of the 16 wavefronts have
