@@ -1047,7 +1047,8 @@ size_t partial_bytes(int64_t n_splits, int64_t rows) {
 // call with the count that 4 rounds would allow and the estimate then takes / with
 // this one: 1233 queries on 5303 keys 315 / 248, 1345 on 8800 (4 KV heads) 474 / 438,
 // 1555 on 9975 (8 heads on 1) 355 / 278). A skewed chunk, half of whose workgroups
-// may see no key, is tried up to twice the splits that one round takes.
+// may see no key, is tried up to twice the splits that one round takes; its context is
+// short, so the size that the longest one of them asks for is kept for all longer ones.
 // Up to kOneSplitKeys keys a chunk stays whole: its output and gate leave in the
 // attention kernel's epilogue, with no partials and no merge. The line is a bound on
 // what a short context asks for, not where the forms cross: first chunks, us per call
@@ -1058,6 +1059,7 @@ size_t partial_bytes(int64_t n_splits, int64_t rows) {
 // walk 16 tiles in a row (8 queries 29.9, 19.9 on 768 keys in 64-key splits).
 constexpr int kMinSplitTiles = 2;  // 64 keys
 constexpr int kMaxRounds = 4;
+constexpr int kRoundTiles = 16;  // tiles of a split past the first round: the estimate never takes fewer
 constexpr int kOneSplitKeys = 512;
 bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
 int64_t max_splits(int64_t n_kv, int64_t wgs, bool skew) {
@@ -1073,8 +1075,9 @@ int64_t max_splits(int64_t n_kv, int64_t wgs, bool skew) {
             const float fill = (float)(i * wgs) / (float)((i * wgs + cus - 1) / cus * cus);
             if (fill > 1.01f * best) best = fill, s = i;
         }
-        const int64_t tries = (cus + wgs - 1) / wgs * 2;
-        if (skew && tries > s) s = tries < rounds ? tries : rounds;
+        const int64_t one = (cus + wgs - 1) / wgs, filled = (n_kv + kRoundTiles * kPK - 1) / (kRoundTiles * kPK);
+        if (!skew && s > one && s > filled) s = one > filled ? one : filled;
+        if (skew) s = 2 * one < rounds ? 2 * one : rounds;
     }
     if (s > by_len) s = by_len;
     if (s > kMaxSplits) s = kMaxSplits;
@@ -1168,7 +1171,7 @@ int64_t split_keys(int64_t n_q, int64_t n_kv, int64_t Hkv, int64_t qb, int64_t q
 // its choice costs 0.4% more than the best count on average, 5% of the shapes lose
 // more than 3%; with the estimate above it was 3.2% and 25%. Host time 1 to 5 us.
 constexpr int kXcds = 8, kEngines = 4, kMaxEngineCus = 16;
-constexpr float kSkewWg = 5.0f, kSkewDead = 0.5f, kSkewMerge = 3.3f, kSkewRow = 0.85e-4f, kSkewMany = 0.6f;
+constexpr float kSkewWg = 5.0f, kSkewDead = 0.5f, kSkewMerge = 3.3f, kSkewRow = 0.85e-4f, kSkewMany = 0.55f;
 // a split chunk has to be clearly ahead of an unsplit one, and a second round of a
 // first one (2000 queries on 4001 keys, 8 on 1: 135 us with 2 splits, 142 with 5)
 constexpr float kSkewMargin = 0.96f, kSkewLate = 1.04f;

@@ -104,7 +104,7 @@ def test_prefill_workspace_of_a_longer_cache_serves_a_shorter_one(sqa, n_q):
         last = need
 
 
-@pytest.mark.parametrize("n_q,n_kv,splits", [(512, 16896, 6), (300, 3328, 20), (2048, 133120, 1), (37, 20224, 42),
+@pytest.mark.parametrize("n_q,n_kv,splits", [(512, 16896, 6), (300, 3328, 13), (2048, 133120, 1), (37, 20224, 42),
                                              (1280, 6400, 4)])
 def test_prefill_workspace_holds_what_the_plan_uses(sqa, n_q, n_kv, splits):
     """Tile records, Q pairs and a mask copy, and partials for the splits that the
