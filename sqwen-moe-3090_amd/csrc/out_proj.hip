@@ -36,6 +36,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kQK = 256;           // values per Q4_K super-block
 constexpr int kBlockBytes = 144;   // bytes per super-block
 constexpr int kGemvTokens = 4;     // token counts up to this take op_gemv
+constexpr int64_t kPrepPairs = 2048;  // 8 wavefronts per CU, see op_prep
 
 __device__ __forceinline__ float h2f(uint32_t bits) {
     _Float16 h;
@@ -45,12 +46,14 @@ __device__ __forceinline__ float h2f(uint32_t bits) {
 }
 
 // ---------------------------------------------------------------- op_prep
-// One wavefront per (16 tokens, 32-value sub-block of K): lane 16q + n takes values
-// 8q .. 8q + 7 of token n and writes xg = x * sigmoid(gate) as fp16 hi and lo in the
-// order in which op_gemm reads them, 1 KB per load. Its time is one chain of load, exp
-// and store; a wavefront per two sub-blocks leaves half as many to overlap: us per
-// call of the whole projection, that / this: 33 tokens, N = 5120, K = 2048 17.3 / 14.6,
-// 100, 8192, 2048 20.1 / 19.2, 300, 4096, 4096 46.6 / 46.0, 512, 2048, 4096 34.0 / 33.7.
+// One wavefront per 16 tokens and SUBS 32-value sub-blocks of K (1, or a pair): lane
+// 16q + n takes values 8q .. 8q + 7 of token n and writes xg = x * sigmoid(gate) as
+// fp16 hi and lo in the order in which op_gemm reads them, 1 KB per load. Its time is
+// one chain of load, exp and store while there are few wavefronts: one sub-block
+// each then (us per call of the whole projection, pairs / this: 33 tokens, N = 5120,
+// K = 2048 17.3 / 14.6, 100, 8192, 2048 20.1 / 19.2, 300, 4096, 4096 46.6 / 46.0), and
+// its stores from kPrepPairs pairs on (512, 2048, 4096 32.3 / 32.5, 2048 of them 105.8 /
+// 106.1).
 // B operand (c, e) of super-block s, c < 4, e < 2, holds in lane 16g + n
 // the values 64g + 32e + 8c .. + 7 of token n: an MFMA then takes from each lane
 // group another code group (64 values, 32 bytes of a weight row), so a lane needs
@@ -69,76 +72,89 @@ __device__ __forceinline__ float xsum32(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <bool GATE, bool VEC>
+template <bool GATE, bool VEC, int SUBS>
 __global__ __launch_bounds__(256) void op_prep_kernel(const char *__restrict__ x, int64_t x_nb1,
                                                       const char *__restrict__ gate, int64_t g_nb1, int K, int M,
                                                       int tiles, uint4 *__restrict__ xb, uint16_t *__restrict__ sb) {
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int subs = K / 32;
+    const int subs = K / 32, per = subs / SUBS;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wid >= (int64_t)tiles * subs) return;
-    const int T = (int)(wid / subs), sub = (int)(wid - (int64_t)T * subs);
-    const int pr = sub >> 1, e = sub & 1;  // sub-block pair (64 values), which of the two
+    if (wid >= (int64_t)tiles * per) return;
+    const int T = (int)(wid / per), sub0 = (int)(wid - (int64_t)T * per) * SUBS;
+    const int pr = sub0 >> 1;  // sub-block pair (64 values)
     const int t = 16 * T + n;
-    float v[8], gv[8];
+    uint32_t sw[SUBS][3];  // the three parts of S
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
-    if (t < M) {
-        const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 32 * sub + 8 * g;
-        const float *gr = GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 32 * sub + 8 * g : nullptr;
-        if (VEC) {
+    for (int u = 0; u < SUBS; ++u) {
+        const int sub = sub0 + u;
+        float v[8], gv[8];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                const float4 a = reinterpret_cast<const float4 *>(xr)[c];
-                v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
-                if (GATE) {
-                    const float4 b = reinterpret_cast<const float4 *>(gr)[c];
-                    gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
+        for (int j = 0; j < 8; ++j) v[j] = gv[j] = 0.0f;
+        if (t < M) {
+            const float *xr = reinterpret_cast<const float *>(x + t * x_nb1) + 32 * sub + 8 * g;
+            const float *gr = GATE ? reinterpret_cast<const float *>(gate + t * g_nb1) + 32 * sub + 8 * g : nullptr;
+            if (VEC) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const float4 a = reinterpret_cast<const float4 *>(xr)[c];
+                    v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
+                    if (GATE) {
+                        const float4 b = reinterpret_cast<const float4 *>(gr)[c];
+                        gv[4 * c] = b.x, gv[4 * c + 1] = b.y, gv[4 * c + 2] = b.z, gv[4 * c + 3] = b.w;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    v[j] = xr[j];
+                    if (GATE) gv[j] = gr[j];
                 }
             }
-        } else {
+            if (GATE) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                v[j] = xr[j];
-                if (GATE) gv[j] = gr[j];
+                for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
             }
         }
-        if (GATE) {
+        float sum = 0.0f;
+        uint16_t hb[8], lb[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (1.0f + expf(-gv[j])));
+        for (int j = 0; j < 8; ++j) {
+            sum += v[j];
+            float a = v[j];
+            // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
+            asm volatile("" : "+v"(a));
+            const _Float16 h = (_Float16)a;
+            const _Float16 l = (_Float16)(a - (float)h);
+            __builtin_memcpy(&hb[j], &h, 2);
+            __builtin_memcpy(&lb[j], &l, 2);
         }
-    }
-    float sum = 0.0f;
-    uint16_t hb[8], lb[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        sum += v[j];
-        float a = v[j];
-        // opaque: one fp32 value feeds both the stored hi and the hi subtracted for lo
-        asm volatile("" : "+v"(a));
-        const _Float16 h = (_Float16)a;
-        const _Float16 l = (_Float16)(a - (float)h);
-        __builtin_memcpy(&hb[j], &h, 2);
-        __builtin_memcpy(&lb[j], &l, 2);
-    }
-    uint4 a, b;
-    __builtin_memcpy(&a, hb, 16);
-    __builtin_memcpy(&b, lb, 16);
-    uint4 *o = xb + ((int64_t)T * subs + 8 * (pr >> 2) + 2 * g + e) * 128 + 16 * (pr & 3) + n;
-    o[0] = a;
-    o[64] = b;
-    // S = its leading 8 bits (truncated) + those of the rest, twice: each
-    // difference is exact
-    float r = xsum32(xsum16(sum));
-    if (g == (pr & 3)) {
-        uint16_t *s = sb + (((int64_t)T * (subs / 8) + (pr >> 2)) * 64 + lane) * 8 + e;
+        uint4 a, b;
+        __builtin_memcpy(&a, hb, 16);
+        __builtin_memcpy(&b, lb, 16);
+        uint4 *o = xb + ((int64_t)T * subs + 8 * (pr >> 2) + 2 * g + (sub & 1)) * 128 + 16 * (pr & 3) + n;
+        o[0] = a;
+        o[64] = b;
+        // S = its leading 8 bits (truncated) + those of the rest, twice: each
+        // difference is exact
+        float r = xsum32(xsum16(sum));
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const uint32_t top = __float_as_uint(r) & 0xFFFF0000u;
-            s[2 * c] = (uint16_t)(top >> 16);
+            sw[u][c] = top >> 16;
             r -= __uint_as_float(top);
         }
-        s[6] = 0;
+    }
+    if (g == (pr & 3)) {
+        uint16_t *s = sb + (((int64_t)T * (subs / 8) + (pr >> 2)) * 64 + lane) * 8;
+        if constexpr (SUBS == 2) {
+            *reinterpret_cast<uint4 *>(s) =
+                make_uint4(sw[0][0] | (sw[1][0] << 16), sw[0][1] | (sw[1][1] << 16), sw[0][2] | (sw[1][2] << 16), 0u);
+        } else {
+            s += sub0 & 1;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) s[2 * c] = (uint16_t)sw[0][c];
+            s[6] = 0;
+        }
     }
 }
 
@@ -769,18 +785,23 @@ int launch_out_proj(const sqa_tensor &w, const sqa_tensor &x, const sqa_tensor *
     const int prof = profile_start("out_proj", s);
     const bool vec = (uintptr_t)x.data % 16 == 0 && x.nb[1] % 16 == 0 &&
                      (!gate || ((uintptr_t)gate->data % 16 == 0 && gate->nb[1] % 16 == 0));
-    const dim3 pg((unsigned)((L.tiles * (K / 32) + 3) / 4));
     const char *xd = (const char *)x.data, *gd = gate ? (const char *)gate->data : nullptr;
     const int64_t xn = (int64_t)x.nb[1], gn = gate ? (int64_t)gate->nb[1] : 0;
     const int Ki = (int)K, Mi = (int)M, tl = (int)L.tiles;
+    const int subs = L.tiles * (K / 64) >= kPrepPairs ? 2 : 1;
+    const dim3 pg((unsigned)((L.tiles * (K / 32) / subs + 3) / 4));
+#define SQA_PREP(GATE, VEC)                                                                       \
+    (subs == 2 ? op_prep_kernel<GATE, VEC, 2> : op_prep_kernel<GATE, VEC, 1>)<<<pg, dim3(256), 0, s>>>( \
+        xd, xn, gd, gn, Ki, Mi, tl, xb, sb)
     if (gate && vec)
-        op_prep_kernel<true, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
+        SQA_PREP(true, true);
     else if (gate)
-        op_prep_kernel<true, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
+        SQA_PREP(true, false);
     else if (vec)
-        op_prep_kernel<false, true><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
+        SQA_PREP(false, true);
     else
-        op_prep_kernel<false, false><<<pg, dim3(256), 0, s>>>(xd, xn, gd, gn, Ki, Mi, tl, xb, sb);
+        SQA_PREP(false, false);
+#undef SQA_PREP
     GemmParams p;
     p.w = (const uint8_t *)w.data;
     p.w_nb1 = (int64_t)w.nb[1];

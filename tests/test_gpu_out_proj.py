@@ -156,3 +156,11 @@ def test_fewer_tokens_take_no_longer(sqa, dev):
     a, b = (sorted(t)[4] for t in times)
     print(f"W_o, 5120 rows: 16 tokens {a:.1f} us, 32 tokens {b:.1f} us")
     assert a <= 1.05 * b
+
+
+@pytest.mark.parametrize("K,M", [(4096, 496), (4096, 497), (4096, 512), (1792, 1169)])
+@pytest.mark.parametrize("gate,unaligned", [(True, False), (True, True), (False, False), (False, True)])
+def test_out_proj_pre_pass_forms(sqa, orc, dev, K, M, gate, unaligned):
+    # both sides of the step from one sub-block per wavefront to pairs (2048 pairs of 16
+    # tokens), 28 pairs a row, every load form
+    assert run(sqa, orc, dev, 64, K, M, 40 + M, gate=gate, unaligned=unaligned, outliers=4) <= TOL
