@@ -1059,7 +1059,7 @@ size_t partial_bytes(int64_t n_splits, int64_t rows) {
 // walk 16 tiles in a row (8 queries 29.9, 19.9 on 768 keys in 64-key splits).
 constexpr int kMinSplitTiles = 2;  // 64 keys
 constexpr int kMaxRounds = 4;
-constexpr int kRoundTiles = 16;  // tiles of a split past the first round: the estimate never takes fewer
+constexpr int kRoundTiles = 16;  // tiles of a split past the first round: the estimate hardly ever takes fewer
 constexpr int kOneSplitKeys = 512;
 bool skewed(int64_t n_q, int64_t n_kv) { return n_kv < 4 * n_q; }
 int64_t max_splits(int64_t n_kv, int64_t wgs, bool skew) {
